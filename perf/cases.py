@@ -1,0 +1,863 @@
+"""What a user of this framework has it do, as timed cases: the path stage on explicit paths, on held path lists (eager
+calls with their gradient and captured steps), the whole-call forward models with path finder and misfit, and single scattering from pair
+tables.
+
+listed() names the cases, draw(rng) gives more of the same ranges, prepare(case, seed) makes what a program holds
+before the call, run(state) is one pass through the public entry points, work(case) counts what the pass cannot do
+without, and exact(case, seed) evaluates the same outputs in 64 bits with plain torch, from the phase file and the
+formulas alone. Structures and path lists are made here (a batched enumeration in torch), so that exact() sees the
+same inputs without the package.
+"""
+from __future__ import annotations
+
+import functools
+import math
+from pathlib import Path
+
+import numpy as np
+import torch
+
+GOLD = Path(__file__).resolve().parents[1] / "tests" / "golden"
+# the phase files the repository's tests and benchmark use: K edges (V in Ge-V; W metal), an L3 and an M5 edge
+PHASES = {"K": GOLD / "validation/A018/phase.pad", "KW": GOLD / "W/phase.pad", "L3": GOLD / "validation/A014/phase.pad",
+          "M5": GOLD / "validation/A009/phase.pad"}
+NPOT = {"K": 2, "KW": 1, "L3": 1, "M5": 2}
+BOHR = 0.52917721067
+ETOK = 0.2624684236075176
+Q18 = np.round(np.arange(0, 18.0 + 1e-9, 0.05), 10)        # the benchmark's output grid, 361 points
+Q16 = np.round(np.arange(0, 16.0 + 1e-9, 0.05), 10)
+
+
+def _dev():
+    return torch.device("cuda" if torch.cuda.is_available() else "cpu")
+
+
+# ---------------------------------------------------------------------------------------------------- the cases
+def listed():
+    return [
+        # an MCP- or notebook-style call of the drop-in stage on a handful of FEFF paths, with their gradient
+        dict(name="stage_few", kind="stage", edge="K", paths=12, legs=4, grad=True, convention="feff", precision=32),
+        # one chunk of the reference's forward model (2048 paths), L3 edge, larch's spline grid, no gradient
+        dict(name="stage_chunk", kind="stage", edge="L3", paths=2048, legs=3, grad=False, convention="larch",
+             precision=32),
+        # refinement of one small cluster: the captured step of a 79-atom Cu cluster with a Debye-Waller factor
+        dict(name="cluster_step", kind="cluster", lattice="fcc", radius=6.0, rmax=5.0, edge="KW", captured=True,
+             precision=32),
+        # the same kind of loop without a graph: a bcc cluster through plan(pos) and autograd
+        dict(name="cluster_call", kind="cluster", lattice="bcc", radius=9.0, rmax=6.0, edge="K", captured=False,
+             precision=32),
+        # an MD trajectory: 64 frames of a 2000-atom box, 16 absorbers each, 2-4 legs, the captured step
+        dict(name="frames_step", kind="frames", cells=10, frames=64, absorbers=16, rmax=4.6, captured=True),
+        # refinement of a whole box: 4000-atom NiO, every fourth Ni an absorber, the captured step with the R-factor
+        dict(name="refine_step", kind="refine", nx=10, ny=10, nz=5, every=4, rmax=5.0, precision=32, captured=True),
+        # the same model in double precision on a smaller box (reference-precision gradients), eager
+        dict(name="refine_double", kind="refine", nx=5, ny=5, nz=5, every=25, rmax=5.0, precision=64, captured=False),
+        # two edges of a disordered alloy, 2-6 legs, one eager call with its gradient
+        dict(name="edges_call", kind="edges", atoms=8000, absorbers=32, rmax=7.0, legs=6),
+        # the reference's forward model as RMC refinement calls it: spectra of copies, the misfit, its gradient
+        dict(name="spectra_call", kind="spectra", cells=6, copies=8, absorbers=8, rmax=5.0, e0=7.0),
+        # new frames of a trajectory from positions to chi per absorber: path finder, plan, forward, as an average over
+        # MD frames calls it (every frame has its own path list)
+        dict(name="trajectory_call", kind="trajectory", cells=10, copies=8, absorbers=16, rmax=5.0),
+        # single scattering of whole configurations from tables, with the position gradient: a trajectory
+        dict(name="pairs_frames", kind="pairs", structure="bcc", cells=10, frames=64, rmax=9.4),
+        # ... and one configuration of a refinement: the NiO box, two scatterer potentials, a general cell
+        dict(name="pairs_box", kind="pairs", structure="nio", nx=10, ny=10, nz=5, frames=1, rmax=9.4),
+    ]
+
+
+def draw(rng):
+    def logint(lo, hi):
+        return int(round(math.exp(rng.uniform(math.log(lo), math.log(hi)))))
+
+    kind = rng.choice(["stage", "stage", "cluster", "frames", "refine", "edges", "spectra", "trajectory", "pairs",
+                       "pairs"])
+    if kind == "stage":
+        return dict(kind=kind, edge=rng.choice(["K", "KW", "L3", "M5"]), paths=logint(1, 3000), legs=rng.randint(2, 6),
+                    grad=rng.random() < 0.6, convention=rng.choice(["feff", "feff", "larch"]),
+                    precision=rng.choice([32, 32, 64]))
+    if kind == "cluster":
+        return dict(kind=kind, lattice=rng.choice(["fcc", "bcc"]), radius=9.0, rmax=round(rng.uniform(4.0, 6.2), 2),
+                    edge=rng.choice(["K", "KW", "L3"]), captured=rng.random() < 0.5, precision=rng.choice([32, 32, 64]))
+    if kind == "frames":
+        return dict(kind=kind, cells=rng.randint(4, 10), frames=logint(1, 64), absorbers=rng.randint(1, 16),
+                    rmax=round(rng.uniform(3.6, 4.6), 2), captured=rng.random() < 0.6)
+    if kind == "refine":
+        double = rng.random() < 0.3
+        return dict(kind=kind, nx=rng.randint(4, 8), ny=rng.randint(4, 7), nz=rng.randint(3, 5),
+                    every=rng.randint(20, 60) if double else rng.randint(4, 40), rmax=round(rng.uniform(3.8, 5.0), 2),
+                    precision=64 if double else 32, captured=rng.random() < 0.5)
+    if kind == "edges":
+        return dict(kind=kind, atoms=rng.randint(3000, 8000), absorbers=rng.randint(1, 32),
+                    rmax=round(rng.uniform(5.5, 7.0), 2), legs=rng.randint(4, 6))
+    if kind == "spectra":
+        return dict(kind=kind, cells=rng.randint(5, 8), copies=rng.randint(1, 16), absorbers=rng.randint(1, 16),
+                    rmax=round(rng.uniform(4.0, 5.2), 2), e0=round(rng.uniform(-4.0, 9.0), 2))
+    if kind == "trajectory":
+        return dict(kind=kind, cells=rng.randint(5, 10), copies=rng.randint(1, 8), absorbers=rng.randint(1, 16),
+                    rmax=round(rng.uniform(4.0, 5.0), 2))
+    if rng.random() < 0.5:
+        return dict(kind="pairs", structure="nio", nx=rng.randint(5, 10), ny=rng.randint(5, 8), nz=rng.randint(5, 7),
+                    frames=1, rmax=round(rng.uniform(6.0, 9.4), 2))
+    return dict(kind="pairs", structure="bcc", cells=rng.randint(7, 10), frames=logint(1, 64),
+                rmax=round(rng.uniform(6.0, 9.4), 2))
+
+
+# ---------------------------------------------------------------------------------------------------- structures
+def _lattice(basis, a, cells):
+    n = (cells,) * 3 if isinstance(cells, int) else tuple(cells)
+    g = np.stack(np.meshgrid(*[np.arange(k) for k in n], indexing="ij"), -1).reshape(-1, 3)
+    return (g[:, None, :] + np.asarray(basis)[None]).reshape(-1, 3) * a, np.asarray(n, float) * a
+
+
+BCC = [[0, 0, 0], [.5, .5, .5]]
+FCC = [[0, 0, 0], [.5, .5, 0], [.5, 0, .5], [0, .5, .5]]
+
+
+def _rocksalt(cells):
+    """Rock salt with NiO's constant: positions, species (0 the metal), box."""
+    fcc, box = _lattice(FCC, 4.18, cells)
+    return (np.concatenate([fcc, fcc + np.array([2.09, 0, 0])]) % box,
+            np.repeat([0, 1], len(fcc)), box)
+
+
+def _packing(n, dmin, seed):
+    """n random points, at the density of Pt30Ni70, no two closer than dmin in their periodic cube: batches of
+    uniform candidates, each kept if it clears every point placed and every earlier candidate of its batch."""
+    L = (n * (0.3 * 195.08 + 0.7 * 58.69) / 6.02214076e23 / 8.9 * 1e24) ** (1 / 3)
+    rng, dev = np.random.default_rng(seed), _dev()
+    pts = torch.zeros(0, 3, dtype=torch.float64, device=dev)
+
+    def near(a, b):
+        d2 = 0.0
+        for c in range(3):
+            v = a[:, None, c] - b[None, :, c]
+            d2 = d2 + (v - L * torch.round(v / L)) ** 2
+        return d2 < dmin * dmin
+    while len(pts) < n:
+        m = min(4 * (n - len(pts)) + 64, 8000) if len(pts) < 0.9 * n else 8000
+        c = torch.tensor(rng.uniform(0, L, (m, 3)), device=dev)
+        if len(pts):
+            c = c[~near(c, pts).any(1)]
+        c = c[~torch.tril(near(c, c), -1).any(1)]
+        pts = torch.cat([pts, c])[:n]
+    return pts.cpu().numpy(), float(L)
+
+
+def _find(pos, box, absorber, frame_atoms, rmax, legs, batch=128):
+    """Every path of 2..legs legs of the absorbers (indices into pos; an absorber's atoms are those of its own block
+    of frame_atoms) with half length at most rmax: (atoms (P, legs - 1), nleg, absorber slot, deg) as numpy, paths of
+    equal leg count together. A path and its reverse are one path of degeneracy 2 (1 if they are the same)."""
+    dev = _dev()
+    P = torch.as_tensor(pos, device=dev, dtype=torch.float64).reshape(-1, frame_atoms, 3)
+    ab = torch.as_tensor(np.asarray(absorber), device=dev)
+    B = None if box is None else torch.as_tensor(np.broadcast_to(np.asarray(box, float), 3).copy(), device=dev)
+    found = {n: [] for n in range(2, legs + 1)}
+    for s in range(0, len(ab), batch):
+        a = ab[s:s + batch]
+        fr, loc = a // frame_atoms, a % frame_atoms
+        rel = P[fr] - P[fr, loc][:, None, :]
+        if B is not None:
+            rel = rel - B * torch.round(rel / B)
+        d = rel.norm(dim=-1)
+        ok = d <= rmax
+        ok[torch.arange(len(a), device=dev), loc] = False
+        C = int(ok.sum(1).max())
+        if C == 0:
+            continue
+        # candidates in index order, then the absorber itself as intermediate C
+        idx = torch.argsort((~ok).to(torch.int8), dim=1, stable=True)[:, :C]
+        live = torch.gather(ok, 1, idx)
+        rc = torch.gather(rel, 1, idx[..., None].expand(-1, -1, 3))
+        rc = torch.cat([rc, torch.zeros_like(rc[:, :1])], 1)
+        live = torch.cat([live, torch.ones_like(live[:, :1])], 1)
+        back = rc.norm(dim=-1)
+        D = (rc[:, :, None] - rc[:, None]).norm(dim=-1)
+        D = torch.where(live[:, :, None] & live[:, None], D, torch.full_like(D, 1e9))
+        idx = torch.cat([idx + (fr * frame_atoms)[:, None], a[:, None]], 1)
+        who, j = torch.nonzero(live[:, :C], as_tuple=True)
+        seq, length = j[:, None], back[who, j]
+        for m in range(1, legs):
+            rev = seq.flip(1)
+            differ = seq != rev
+            first = differ.to(torch.int8).argmax(1, keepdim=True)
+            pal = ~differ.any(1)
+            keep = (seq[:, -1] != C) & (pal | (seq.gather(1, first) < rev.gather(1, first))[:, 0])
+            keep &= length + back[who, seq[:, -1]] <= 2 * rmax
+            found[m + 1].append((torch.gather(idx[who[keep]], 1, seq[keep]), who[keep] + s,
+                                 torch.where(pal[keep], 1.0, 2.0)))
+            if m == legs - 1:
+                break
+            tot = length[:, None] + D[who, seq[:, -1]]
+            grow = tot + back[who] <= 2 * rmax
+            grow[torch.arange(len(seq), device=dev), seq[:, -1]] = False
+            i, j = torch.nonzero(grow, as_tuple=True)
+            seq, length, who = torch.cat([seq[i], j[:, None]], 1), tot[i, j], who[i]
+    atoms, nleg, slot, deg = [], [], [], []
+    for n, rows in found.items():
+        for at, sl, dg in rows:
+            atoms.append(torch.nn.functional.pad(at, (0, legs - n)))
+            nleg.append(torch.full_like(sl, n))
+            slot.append(sl)
+            deg.append(dg)
+    return tuple(torch.cat(v).cpu().numpy() for v in (atoms, nleg, slot, deg))
+
+
+def _path_list(pos, box, absorber, frame_atoms, rmax, legs, ipot, segment):
+    """The list of every absorber as a plan takes it; ipot (N,) of every atom, segment (A,) of every absorber."""
+    atoms, nleg, slot, deg = _find(pos, box, absorber, frame_atoms, rmax, legs)
+    ab = np.asarray(absorber)[slot]
+    ipots = np.zeros((len(nleg), legs), np.int64)
+    for j in range(1, legs):
+        a = atoms[:, j - 1]
+        ipots[:, j] = np.where(j < nleg, np.where(a == ab, 0, np.asarray(ipot)[a]), 0)
+    return dict(atoms=atoms, nleg=nleg, absorber=ab, ipots=ipots, deg=deg, segment=np.asarray(segment)[slot])
+
+
+def _join(lists):
+    return {k: np.concatenate([x[k] for x in lists]) for k in lists[0]}
+
+
+def _inputs(case, seed, few=False):
+    """The structure of a list case and its path list: dict(pos, box, cell, list, nseg, phases, q, ...). few: a few
+    absorbers only (what work() counts from)."""
+    rng = np.random.default_rng([seed, 77])
+    kind = case["kind"]
+    if kind == "cluster":
+        a = 3.61 if case["lattice"] == "fcc" else 2.87
+        n = int(math.ceil(case["radius"] / a)) + 1
+        pos, _ = _lattice(FCC if case["lattice"] == "fcc" else BCC, a, 2 * n)
+        pos = pos - n * a
+        pos = pos[np.argsort(np.linalg.norm(pos, axis=1), kind="stable")]
+        pos = pos[np.linalg.norm(pos, axis=1) <= case["radius"] + 1e-9]
+        pos = pos + rng.normal(0, 0.05, pos.shape)
+        lst = _path_list(pos, None, [0], len(pos), case["rmax"], 4, np.full(len(pos), NPOT[case["edge"]]), [0])
+        return dict(pos=pos, box=None, cell=None, list=lst, nseg=1, edges=[case["edge"]], q=Q16, slots=1, total=1,
+                    sigma2=0.003)
+    if kind in ("frames", "spectra", "trajectory"):
+        pos0, box = _lattice(BCC, 2.87, case["cells"])
+        F = case["frames"] if kind == "frames" else case["copies"]
+        n, A = len(pos0), case["absorbers"]
+        total = F * A
+        F = 1 if few else F
+        pos = (pos0[None] + rng.normal(0, 0.07, (F, n, 3))).astype(np.float32).astype(float)
+        ab = np.stack([rng.choice(n, A, replace=False) for _ in range(F)])
+        if kind == "trajectory":            # the same absorbers in every frame, one spectrum each, 3 and 4 legs
+            ab[:] = ab[0]
+        flat = (ab + n * np.arange(F)[:, None]).reshape(-1)
+        rows = np.arange(F * A) if kind == "trajectory" else np.repeat(np.arange(F), A)
+        lst = _path_list(pos.reshape(-1, 3), box, flat, n, case["rmax"], 4, np.full(F * n, 2), rows)
+        if kind == "trajectory":
+            lst = {k: v[lst["nleg"] >= 3] for k, v in lst.items()}
+        return dict(pos=pos.reshape(-1, 3), box=box, cell=float(box[0]), list=lst, nseg=int(rows[-1]) + 1,
+                    edges=["K"], q=Q18, n=n,
+                    absorbers=ab, slots=F * A, total=total, sigma2=None)
+    if kind == "refine":
+        pos0, species, box = _rocksalt((case["nx"], case["ny"], case["nz"]))
+        pos = pos0 + rng.normal(0, 0.1, pos0.shape)
+        ab = np.nonzero(species == 0)[0][::case["every"]]
+        total = len(ab)
+        ab = ab[:16] if few else ab
+        lst = _path_list(pos, box, ab, len(pos), case["rmax"], 4, np.where(species == 0, 2, 1), np.arange(len(ab)))
+        return dict(pos=pos, box=box, cell=np.diag(box), list=lst, nseg=len(ab), edges=["K"], q=Q18, slots=len(ab),
+                    total=total, sigma2=None)
+    # edges: half of the absorbers at the L3 edge of the heavy species, half at the K edge of the light one
+    n, A = case["atoms"], case["absorbers"]
+    pos, L = _packing(n, 2.3, [seed, 5])
+    heavy = np.zeros(n, bool)
+    heavy[rng.choice(n, int(0.3 * n), replace=False)] = True
+    lists = []
+    for e, (mask, ip) in enumerate(((heavy, np.ones(n, int)), (~heavy, np.where(heavy, 1, 2)))):
+        ab = rng.choice(np.nonzero(mask)[0], A, replace=False)
+        lst = _path_list(pos, L, ab, n, case["rmax"], case["legs"], ip, e * A + np.arange(A))
+        lst["edge"] = np.full(len(lst["nleg"]), e)
+        lists.append(lst)
+    return dict(pos=pos, box=np.full(3, L), cell=L, list=_join(lists), nseg=2 * A, edges=["L3", "K"], q=Q18,
+                slots=2 * A, total=2 * A, sigma2=None)
+
+
+def _weights(nseg, q, seed):
+    """An upstream gradient of chi (nseg, NK): k^2-weighted noise, as a k^2-weighted misfit of one spectrum gives."""
+    return np.random.default_rng([seed, 9]).normal(size=(nseg, len(q))) * q ** 2
+
+
+def _target(nseg, q, seed):
+    """A data spectrum per segment: three damped shells with noise-free random distances and amplitudes."""
+    r = np.random.default_rng([seed, 10])
+    R = np.array([2.1, 2.95, 4.2])[None, :, None] + r.normal(0, 0.05, (nseg, 3, 1))
+    A = np.array([6.0, 4.0, 8.0])[None, :, None] * (1 + r.normal(0, 0.1, (nseg, 3, 1)))
+    k = np.maximum(q, 0.1)[None, None]
+    return (A * np.sin(2 * k * R + 0.3 * k) * np.exp(-2 * 0.006 * k ** 2 - 2 * R / 9.0) / (k * R ** 2)).sum(1) * (q > 0)
+
+
+WINDOW = dict(kmin=3.0, kmax=16.0, dk=1.0, kweight=2, rmin=1.0, rmax=5.0)
+
+
+def _walks(case, seed):
+    """Explicit paths as a drop-in caller has them: random walks over a displaced bcc lattice (first two shells)."""
+    rng = np.random.default_rng([seed, 3])
+    pos0, box = _lattice(BCC, 2.87, 6)
+    pos = pos0 + rng.normal(0, 0.07, pos0.shape)
+    v = pos0[:, None] - pos0[None]
+    v -= box * np.round(v / box)
+    d = np.linalg.norm(v, axis=-1)
+    nbr = np.argsort(np.where(d < 1e-6, 1e9, d), 1, kind="stable")[:, :14]
+    B, n = case["paths"], case["legs"]
+    seq = np.zeros((B, n), np.int64)
+    seq[:, 0] = rng.integers(0, len(pos), B)
+    for j in range(1, n):
+        nxt = nbr[seq[:, j - 1], rng.integers(0, 14, B)]
+        while j == n - 1 and (nxt == seq[:, 0]).any():       # the last atom is a scatterer
+            bad = np.nonzero(nxt == seq[:, 0])[0]
+            nxt[bad] = nbr[seq[bad, j - 1], rng.integers(0, 14, len(bad))]
+        seq[:, j] = nxt
+    rel = pos[seq] - pos[seq[:, :1]]
+    rel -= box * np.round(rel / box)
+    ipots = np.where(seq == seq[:, :1], 0, 1 + seq % NPOT[case["edge"]])
+    up = rng.normal(size=(B, len(Q18))) * Q18 ** 2
+    return rel, ipots, up
+
+
+def _pair_inputs(case, seed):
+    rng = np.random.default_rng([seed, 21])
+    if case["structure"] == "bcc":
+        pos0, box = _lattice(BCC, 2.87, case["cells"])
+        ipot, cell = np.full(len(pos0), 2), float(box[0])
+    else:
+        pos0, species, box = _rocksalt((case["nx"], case["ny"], case["nz"]))
+        ipot, cell = np.where(species == 0, 2, 1), np.diag(box)
+    pos = pos0[None] + rng.normal(0, 0.08, (case["frames"],) + pos0.shape)
+    return pos, ipot, cell, box, rng.normal(size=len(Q18)) * Q18 ** 2
+
+
+# ---------------------------------------------------------------------------------------------------- the product
+def prepare(case, seed):
+    from feffgpu_amd import GPUPathStage, PathPlan
+    from feffgpu_amd.forward import MultipleScattering, PathSpectra
+    from feffgpu_amd.graph import CapturedStep
+    from feffgpu_amd.pairs import PairTables
+    from feffgpu_amd.transform import FitWindow, RFactorLoss
+    dev, kind = torch.device("cuda"), case["kind"]
+    if kind == "stage":
+        rel, ipots, up = _walks(case, seed)
+        dt = torch.complex64 if case["precision"] == 32 else torch.complex128
+        st = GPUPathStage(str(PHASES[case["edge"]]), device=dev, dtype=dt)
+        return dict(kind=kind, case=case, stage=st, coords=torch.tensor(rel, device=dev, requires_grad=case["grad"]),
+                    ipots=torch.tensor(ipots, device=dev), up=torch.tensor(up, device=dev, dtype=st.rdtype))
+    if kind == "pairs":
+        pos, ipot, cell, _, up = _pair_inputs(case, seed)
+        pt = PairTables(str(PHASES["K"]), Q18, box=cell, rmax=case["rmax"], device=dev)
+        pt.ipot = torch.tensor(ipot, device=dev)
+        return dict(kind=kind, tables=pt, pos=torch.tensor(pos, device=dev, requires_grad=True),
+                    up=torch.tensor(up, device=dev))
+    I = _inputs(case, seed)
+    pos = torch.tensor(I["pos"], device=dev)
+    if kind == "spectra":
+        ps = PathSpectra(str(PHASES["K"]), Q18, _target(1, Q18, seed)[0], case["e0"], window=(3.0, 16.0),
+                         r_range=(1.0, 5.0), box=I["cell"], rmax=case["rmax"], nlegmax=4, critpw=0.0, device=dev)
+        ps.refresh(I["pos"].reshape(case["copies"], -1, 3), I["absorbers"], np.full(I["n"], 2))
+        return dict(kind=kind, spectra=ps, pos=pos.requires_grad_())
+    if kind == "trajectory":
+        ms = MultipleScattering(str(PHASES["K"]), Q18, 0.0, I["cell"], rmax=case["rmax"], critpw=0.0, device=dev)
+        return dict(kind=kind, ms=ms, pos=pos.reshape(case["copies"], -1, 3),
+                    ipot=torch.full((I["n"],), 2, device=dev), absorbers=torch.tensor(I["absorbers"][0], device=dev))
+    L = I["list"]
+    plan = PathPlan([str(PHASES[e]) for e in I["edges"]], I["q"], L["atoms"], L["nleg"], L["absorber"], L["ipots"],
+                    L["deg"], segment=L["segment"], nseg=I["nseg"], edge=L.get("edge"), sigma2=I["sigma2"],
+                    cell=I["cell"], precision=case.get("precision", 32), device=dev)
+    if case.get("captured"):
+        target = torch.tensor(_target(I["nseg"], I["q"], seed), device=dev)
+        if kind == "refine":
+            loss = RFactorLoss(target, I["q"], FitWindow(**WINDOW), scale=1.0, device=dev)
+        else:
+            w = torch.tensor(I["q"] ** 2, device=dev)
+            loss = lambda seg: 2 * w * (seg - target)       # noqa: E731  a k^2-weighted least-squares misfit
+        step = CapturedStep(plan, len(I["pos"]), loss_grad=loss)
+        return dict(kind="step", step=step, pos=pos, loss=loss if kind == "refine" else None)
+    return dict(kind="call", plan=plan, pos=pos.requires_grad_(),
+                up=torch.tensor(_weights(I["nseg"], I["q"], seed), device=dev))
+
+
+def run(s):
+    kind = s["kind"]
+    if kind == "stage":
+        st, c = s["stage"], s["case"]
+        cchi, reff = st.cchi(s["coords"], s["ipots"])
+        chi = st.chi_fine(cchi, reff, Q18, None, c["convention"])
+        out = [torch.view_as_real(cchi.detach()), reff.detach(), chi.detach()]
+        if c["grad"]:
+            out.append(torch.autograd.grad(chi, s["coords"], s["up"])[0])
+        return out
+    if kind == "trajectory":
+        s["ms"].enumerate(s["pos"], s["ipot"], s["absorbers"])
+        return s["ms"].full_pass(s["pos"].reshape(-1, 3))
+    if kind == "pairs":
+        chi = s["tables"].single_scattering(s["pos"])
+        return [chi.detach(), torch.autograd.grad(chi, s["pos"], s["up"])[0]]
+    if kind == "spectra":
+        chi = s["spectra"].spectra(s["pos"])
+        mis = s["spectra"].misfit(chi.mean(0))
+        return [chi.detach(), mis.detach(), torch.autograd.grad(mis, s["pos"])[0]]
+    if kind == "step":
+        seg, grad = s["step"](s["pos"])
+        return [seg, grad] + ([s["loss"].rfac] if s["loss"] is not None else [])
+    seg, _ = s["plan"](s["pos"])
+    return [seg.detach(), torch.autograd.grad(seg, s["pos"], s["up"])[0]]
+
+
+# ---------------------------------------------------------------------------------------------------- the work
+@functools.lru_cache(maxsize=64)
+def _path_work(key):
+    """(algorithmic flops, paths, atoms, segments, points) of one forward evaluation of a list case, from the paths of
+    a few of its absorbers."""
+    from feffgpu_amd.pad import read_phase_pad
+    from feffgpu_amd.roofline import FLOPS_PER_CMAC, path_cmacs
+    from feffgpu_amd.tables import edge_tables, energies_needed
+    case = {k: v for k, v in key}
+    I = _inputs(case, 0, few=True)
+    L, scale = I["list"], I["total"] / I["slots"]
+    fl = 0.0
+    for e, name in enumerate(I["edges"]):
+        sel = L["edge"] == e if "edge" in L else slice(None)
+        P = read_phase_pad(PHASES[name])
+        T = edge_tables(P, energies_needed(P, I["q"]))
+        fl += path_cmacs(T, L["nleg"][sel], L["ipots"][sel]).sum() * FLOPS_PER_CMAC
+    n = len(I["pos"])
+    if case["kind"] in ("frames", "spectra", "trajectory"):     # a few absorbers: those of the first copy
+        n *= case.get("frames", case.get("copies"))
+    return fl * scale, len(L["nleg"]) * scale, n, I["nseg"] * scale, len(I["q"])
+
+
+def work(case):
+    """The forward's algorithmic operations, three times over with a gradient (its adjoint counts twice the forward);
+    bytes: positions, the path list and the upstream gradient read, chi and the position gradient written."""
+    kind, nk = case["kind"], len(Q18)
+    if kind == "stage":
+        from feffgpu_amd.pad import read_phase_pad
+        from feffgpu_amd.roofline import FLOPS_PER_CMAC, path_cmacs
+        from feffgpu_amd.tables import edge_tables
+        _, ipots, _ = _walks(case, 0)
+        T = edge_tables(read_phase_pad(PHASES[case["edge"]]))
+        B, n, b = case["paths"], case["legs"], case["precision"] // 8
+        fl = path_cmacs(T, np.full(B, n), ipots).sum() * FLOPS_PER_CMAC
+        by = B * (n * 32 + 2 * T.E * b + b + nk * b)
+        return {"bytes": by + (B * (nk * b + n * 24) if case["grad"] else 0), "flops": fl * (3 if case["grad"] else 1)}
+    if kind == "pairs":
+        n = 2 * case["cells"] ** 3 if case["structure"] == "bcc" else 8 * case["nx"] * case["ny"] * case["nz"]
+        nr, npot = int(round((case["rmax"] - 1.5) / 0.002)) + 1, NPOT["K"]
+        # every unordered pair's distance once (about 20 operations) and the tables read by the sum and its adjoint
+        return {"bytes": case["frames"] * n * 48 + 2 * npot * nr * nk * 4 + nk * 16,
+                "flops": 20 * case["frames"] * n * (n - 1) / 2 + 4 * npot * nr * nk}
+    key = tuple(sorted((k, v) for k, v in case.items() if k != "name"))
+    fl, P, n, nseg, nk = _path_work(key)
+    grad = kind != "trajectory"
+    by = n * (48 if grad else 24) + P * 40 + nseg * nk * (16 if grad else 4)
+    return {"bytes": int(by), "flops": (3 if grad else 1) * fl}
+
+
+# ---------------------------------------------------------------------------------------------------- in 64 bits
+class _Phase:
+    """A phase.pad file and the tables of the path amplitude, read and built here in FP64."""
+
+    def __init__(self, file, dev):
+        lines = Path(file).read_text(encoding="latin-1").splitlines()
+        nsp, ne, ne1, _, nph, ihole, _, npack, _ = (int(lines[0][1 + 5 * j:5 + 5 * j]) for j in range(9))
+        at = 1
+
+        def packed(width, count):
+            nonlocal at
+            rows, have = [], 0
+            while have < count:
+                s = lines[at].rstrip()
+                at += 1
+                n = min(len(s) // width, count - have)
+                if n > 0:
+                    rows.append(np.frombuffer(s[1:1 + n * width].encode("latin-1"), np.uint8).reshape(n, width))
+                    have += n
+            return np.concatenate(rows).astype(np.int64) - 37
+
+        def number(c):
+            m = (c[:, 1] // 2) / 90.0 ** 2 + sum(c[:, i] / 90.0 ** (i + 1) for i in range(2, npack))
+            return 180.0 * np.where(c[:, 1] % 2 == 1, 1.0, -1.0) * m * 10.0 ** (c[:, 0] - 45.0)
+
+        def cplx(count):
+            c = packed(2 * npack, count)
+            return number(c[:, :npack]) + 1j * number(c[:, npack:])
+
+        edge = number(packed(npack, 3))[2]
+        em, eref = cplx(ne), cplx(ne)
+        shifts = []
+        for _ in range(nph + 1):
+            l0 = int(lines[at][1:4])
+            at += 1
+            shifts.append(cplx(ne * (2 * l0 + 1)).reshape(ne, 2 * l0 + 1)[:ne1])
+        rkk = cplx(ne * 8).reshape(8, ne).T[:ne1]
+        e = em.real[:ne1] - edge
+        self.E = ne1
+        xk, ck = np.sign(e) * np.sqrt(np.abs(2 * e)), np.sqrt(2 * (em - eref))[:ne1]
+        self.kf = xk / BOHR
+        L = max(s.shape[1] // 2 for s in shifts)
+        lmax = np.zeros((nph + 1, ne1), int)
+        tl = np.zeros((nph + 1, ne1, L + 1), complex)         # index l = il - 1
+        for p, s in enumerate(shifts):
+            l0 = s.shape[1] // 2
+            big = np.abs(np.sin(s[:, l0:])) > 1e-7
+            lmax[p] = np.where(big.any(1), l0 - np.argmax(big[:, ::-1], 1), 0)
+            l = np.arange(l0 + 1)
+            t = (np.exp(2j * s) - 1) / 2j
+            tl[p, :, :l0 + 1] = t[:, l0 - l] * (l + 1) + t[:, l0 + l] * l
+        self.il = int(lmax.max()) + 1
+        kappa = {1: -1, 4: -2, 9: -3}[ihole]
+        self.ilinit = {1: 1, 4: 2, 9: 3}[ihole]
+        self.chan = {}
+        for i, kap in enumerate((kappa - 1, -kappa, kappa + 1)):
+            lk = kap if kap > 0 else -kap - 1
+            if 0 <= lk <= 4 and kap != 0:
+                self.chan[lk + 1] = self.chan.get(lk + 1, 0) - rkk[:, i] ** 2 / (2 * lk + 1) / 3
+        c = lambda a: torch.tensor(a, device=dev)       # noqa: E731
+        self.ck, self.dk = c(ck), c(ck - xk)
+        self.lmax, self.tl = c(lmax), c(np.ascontiguousarray(tl[:, :, :self.il]))
+        self.chan = {k: c(v) for k, v in self.chan.items()}
+        self.sets = {}
+        self.dev = dev
+
+    def lam(self, n):
+        """(m, n) of the lambda set of an n-leg path, the first L0 its final-state part: (M, N, L0)."""
+        if n > 2:
+            M, N = [0, -1, 1, 0, -2, 2], [0, 0, 0, 1, 0, 0]
+            return M, N, 4 if self.ilinit == 1 else 6
+        s, i = [], self.ilinit
+        for nn in range(i + 1):
+            for m in range(i + 1):
+                if 2 * nn + m <= 3 * i:
+                    s += [(x, nn) for x in ((0,) if m == 0 else (-m, m))]
+        s = s[:15]
+        return [m for m, _ in s], [x for _, x in s], len(s)
+
+
+def _grid(kf, q, convention):
+    """Interpolation matrix (len(q), E), q clamped to the phase grid: linear, or the not-a-knot cubic spline."""
+    E, x = len(kf), np.clip(q, kf[0], kf[-1])
+    j = np.clip(np.searchsorted(kf, x, side="right") - 1, 0, E - 2)
+    h = np.diff(kf)
+    f = (x - kf[j]) / h[j]
+    S, I = np.zeros((len(q), E)), np.eye(E)
+    if convention == "feff":
+        S[np.arange(len(q)), j], S[np.arange(len(q)), j + 1] = 1 - f, f
+        return S
+    A, R = np.zeros((E, E)), np.zeros((E, E))           # second derivatives m: A m = R y
+    for i in range(1, E - 1):
+        A[i, i - 1:i + 2] = h[i - 1], 2 * (h[i - 1] + h[i]), h[i]
+        R[i, i - 1:i + 2] = 6 / h[i - 1], -6 / h[i - 1] - 6 / h[i], 6 / h[i]
+    A[0, :3] = h[1], -h[0] - h[1], h[0]
+    A[-1, -3:] = h[-1], -h[-2] - h[-1], h[-2]
+    M = np.linalg.solve(A, R)
+    hj, f = h[j][:, None], f[:, None]
+    return (1 - f) * I[j] + f * I[j + 1] + hj ** 2 / 6 * (((1 - f) ** 3 - (1 - f)) * M[j] + (f ** 3 - f) * M[j + 1])
+
+
+def _rotation(beta, M, ilmax):
+    """d^l_{m1 m2}(beta) (P, ilmax, len(M), len(M)) for l = 0..ilmax-1: the explicit sum at l = max(|m1|, |m2|), then
+    the three-term recursion in l; times xnlm(l, |m1|) (-1)^m1 / xnlm(l, |m2|)."""
+    dev, P, n = beta.device, beta.shape[0], len(M)
+    c, ch, sh = torch.cos(beta)[:, None], torch.cos(beta / 2), torch.sin(beta / 2)
+    F = math.factorial
+    seed = {}
+    for a, m1 in enumerate(M):
+        for b, m2 in enumerate(M):
+            j, v = max(abs(m1), abs(m2)), 0.0
+            for s in range(2 * j + 1):
+                d = (j + m2 - s, s, m1 - m2 + s, j - m1 - s)
+                if min(d) < 0:
+                    continue
+                w = math.sqrt(F(j + m1) * F(j - m1) * F(j + m2) * F(j - m2)) / math.prod(F(x) for x in d)
+                t = (-1.0) ** (m1 - m2 + s) * w * torch.ones(P, dtype=torch.float64, device=dev)
+                for _ in range(2 * j + m2 - m1 - 2 * s):
+                    t = t * ch
+                for _ in range(m1 - m2 + 2 * s):
+                    t = t * sh
+                v = v + t
+            seed.setdefault(j, []).append((a * n + b, v))
+    m1, m2 = np.repeat(M, n).astype(float), np.tile(M, n).astype(float)
+    start = np.maximum(np.abs(m1), np.abs(m2))
+    prev, cur = (torch.zeros(P, n * n, dtype=torch.float64, device=dev) for _ in range(2))
+    rows = []
+    T = lambda v: torch.tensor(v, device=dev)       # noqa: E731
+    for l in range(ilmax):
+        if l == 1:
+            nxt = torch.where(T(start < 1), c.expand(P, n * n), torch.zeros_like(cur))
+        elif l > 1:
+            k = l - 1
+            on = start <= k
+            den = np.where(on, k * np.sqrt(np.maximum((l * l - m1 ** 2) * (l * l - m2 ** 2), 1e-300)), 1.0)
+            pa = np.where(on, (2 * k + 1) * k * l / den, 0.0)
+            qa = np.where(on, (2 * k + 1) * m1 * m2 / den, 0.0)
+            ra = np.where(on, l * np.sqrt(np.maximum((k * k - m1 ** 2) * (k * k - m2 ** 2), 0.0)) / den, 0.0)
+            nxt = (T(pa) * c - T(qa)) * cur - T(ra) * prev
+        else:
+            nxt = torch.zeros_like(cur)
+        if l in seed:
+            pos = [p for p, _ in seed[l]]
+            nxt = nxt.index_copy(1, T(np.array(pos)), torch.stack([v for _, v in seed[l]], 1))
+        prev, cur = cur, nxt
+        xa, xb = (np.array([math.sqrt((2 * l + 1) * math.exp(math.lgamma(l - a + 1) - math.lgamma(l + a + 1)))
+                            if a <= l else 0.0 for a in np.abs(m).astype(int)]) for m in (m1, m2))
+        rows.append(nxt * T(np.where(xb > 0, xa * (-1) ** np.abs(m1) / np.where(xb > 0, xb, 1.0), 0.0)))
+    return torch.stack(rows, 1).reshape(P, ilmax, n, n)
+
+
+def _waves(z, ilmax, cols, lx):
+    """Spherical-wave factors c[il][im] (P, E, ilmax, cols) of a leg, zero beyond its lx rows as FEFF has them."""
+    one, zero = torch.ones_like(z), torch.zeros_like(z)
+    rows, diag = [], [one]
+    for m in range(1, cols):
+        diag.append(diag[-1] * z * -(2 * m - 1))
+    for r in range(1, ilmax + 1):
+        row = []
+        for im in range(1, cols + 1):
+            if r < im:
+                v = zero
+            elif r == im:
+                v = diag[im - 1]
+            elif r == im + 1:
+                v = diag[im - 1] * (one - z * im) * (2 * im - 1)
+            else:
+                p = rows[-1][im - 1] + (rows[-1][im - 2] if im > 1 else 0)
+                v = rows[-2][im - 1] - (2 * r - 3) * z * p
+            row.append(v if (im == 1 and r <= 2) else torch.where(lx >= r, v, zero))
+        rows.append(row)
+    return torch.stack([torch.stack(r, -1) for r in rows], -2)
+
+
+def _trig(v):
+    r, s2 = v.norm(dim=-1), v[..., 0] ** 2 + v[..., 1] ** 2
+    flat = s2 < 1e-12
+    rxy = torch.sqrt(torch.where(flat, torch.ones_like(s2), s2))
+    ct = v[..., 2] / r
+    st = torch.where(flat, torch.zeros_like(r), rxy / r)
+    cp = torch.where(flat, torch.where(ct < 0, -1.0, 1.0).to(r), v[..., 0] / rxy)
+    sp = torch.where(flat, torch.zeros_like(r), v[..., 1] / rxy)
+    return ct, st, cp, sp
+
+
+def _angle(x, y, fi):
+    x = torch.where(x.abs() < 1e-6, torch.zeros_like(x), x)
+    y = torch.where(y.abs() < 1e-6, torch.zeros_like(y), y)
+    both = (x == 0) & (y == 0)
+    return torch.where(both, fi, torch.atan2(y, torch.where(both, torch.ones_like(x), x)))
+
+
+def _cchi(ph, coords, ipots):
+    """cchi (P, E) and reff (P,) A of paths of one leg count: coords (P, n, 3) A, absorber first."""
+    P, n, _ = coords.shape
+    E, IL, dev = ph.E, ph.il, coords.device
+    rat = torch.cat([coords, coords[:, :1]], 1) / BOHR
+    vin = rat[:, 1:] - rat[:, :-1]                      # leg J = 1..n at index J - 1
+    vout = torch.cat([vin[:, 1:], vin[:, :1]], 1)
+    r = vin.norm(dim=-1)
+    (pct, pst, pcp, psp), (qct, qst, qcp, qsp) = _trig(vout), _trig(vin)
+    cpp, spp = qcp * pcp + qsp * psp, psp * qcp - pcp * qsp
+    phi, phip = torch.atan2(qsp, qcp), torch.atan2(psp, pcp)
+    alpha = _angle(-(qst * pct - qct * pst * cpp), pst * spp, phip - phi)
+    gamma = _angle(-(qst * pct * cpp - qct * pst), -qst * spp, torch.zeros_like(phi))
+    u1 = torch.stack([qst * qcp, qst * qsp, qct], -1)
+    u2 = torch.stack([pst * pcp, pst * psp, pct], -1)
+    cr = torch.linalg.cross(u1, u2)
+    beta = torch.atan2(torch.sqrt((cr ** 2).sum(-1) + 1e-30), (qct * pct + qst * pst * cpp).clamp(-1, 1))
+    alpha, gamma = math.pi - gamma, math.pi - alpha
+    eta = torch.cat([alpha[:, -1:], alpha[:, :-1]], 1) + gamma
+    M, N, L0 = ph.lam(n)
+    L = len(M)
+    cols = max(max(abs(m) + k for m, k in zip(M, N)), max(N)) + 1
+    atom = torch.cat([ipots, ipots[:, :1]], 1)
+    lx = torch.maximum(ph.lmax[atom[:, 1:]], ph.lmax[atom[:, :-1]]) + 1      # (P, n, E)
+    W = _rotation(beta.reshape(-1), M, IL).reshape(P, n, IL, L, L)
+    c = [_waves(-1j / (ph.ck * r[:, J, None]), IL, cols, lx[:, J]) for J in range(n)]
+    phase = [torch.exp(-1j * eta[:, J, None] * torch.tensor(M, device=dev, dtype=torch.float64)) for J in range(n)]
+    groups = {}
+    for i in range(L):
+        for j in range(L):
+            groups.setdefault((abs(M[i]) + N[i], N[j]), []).append(i * L + j)
+
+    def matrix(X, Y, w, J, rows):
+        """sum over il of X Y w W for every (lambda1, lambda2), with the row phase of leg J: (P, E, L, L)"""
+        parts, where = [], []
+        Wf = W[:, J - 1 if rows is None else J, :, :, :].reshape(P, IL, L * L)
+        for (a, b), idx in groups.items():
+            Z = X[..., a] * Y[..., b] * w
+            V = torch.cat([Z.real, Z.imag], 1).contiguous()
+            V = torch.bmm(V, Wf[:, :, idx].contiguous())
+            parts.append(torch.complex(V[:, :E], V[:, E:]))
+            where += idx
+        out = torch.cat(parts, -1)[..., torch.tensor(np.argsort(where), device=dev)].reshape(P, E, L, L)
+        return out * phase[0 if rows is not None else J][:, None, :, None]
+
+    def product(A, B):
+        return (A[..., :, :, None] * B[..., None, :, :]).sum(-2)
+    w = torch.zeros(E, IL, dtype=torch.complex128, device=dev)
+    for il, v in ph.chan.items():
+        w[:, il - 1] = v * (2 * il - 1)
+    U = matrix(c[0], c[n - 1], w, n - 1, "termination")[..., :L0, :L0]
+    il = torch.arange(1, IL + 1, device=dev)
+    for s in range(n - 1, 0, -1):
+        t = ph.tl[ipots[:, s]] * (il <= ph.lmax[ipots[:, s]][..., None] + 1)
+        F = matrix(c[s], c[s - 1], t, s, None)
+        U = product(U, F[..., :L0 if s == n - 1 else L, :L0 if s == 1 else L])
+    R = r.sum(1)
+    cfac = torch.exp(1j * R[:, None] * ph.dk) / (ph.ck ** n * r.prod(1)[:, None])
+    return U.diagonal(dim1=-2, dim2=-1).sum(-1) * cfac, R * BOHR / 2
+
+
+def _chi(cchi, reff, S, q, sigma2):
+    amp = torch.sqrt(cchi.real ** 2 + cchi.imag ** 2 + 1e-30)
+    ang = torch.atan2(cchi.imag, cchi.real)
+    d = torch.diff(ang, dim=-1)
+    d = d - 2 * math.pi * torch.round(d.detach() / (2 * math.pi))
+    ang = torch.cat([ang[:, :1], ang[:, :1] + torch.cumsum(d, -1)], -1)
+    chi = (amp @ S.T) * torch.sin(ang @ S.T + 2 * q * reff[:, None])
+    return chi if sigma2 is None else chi * torch.exp(-2 * sigma2 * q * q)
+
+
+def _list_exact(I, q, loss_grad):
+    """(chi_seg, dL/dpos) of a list in FP64, dL/dchi_seg from loss_grad(chi_seg); without a loss_grad chi_seg alone."""
+    dev, L = _dev(), I["list"]
+    nleg, edge = L["nleg"], L.get("edge", np.zeros(len(L["nleg"]), int))
+    pos = torch.tensor(I["pos"], device=dev)
+    box = None if I["box"] is None else torch.tensor(I["box"], device=dev)
+    qt = torch.tensor(q, device=dev)
+    T = {k: torch.tensor(L[k], device=dev) for k in ("atoms", "absorber", "ipots", "deg", "segment")}
+    seg = torch.zeros(I["nseg"], len(q), dtype=torch.float64, device=dev)
+    chunks = []
+    for e, name in enumerate(I["edges"]):
+        ph = _Phase(PHASES[name], dev)
+        S = torch.tensor(_grid(ph.kf, q, "feff"), device=dev)
+        for n in np.unique(nleg):
+            idx = np.nonzero((nleg == n) & (edge == e))[0]
+            size = 4096 if dev.type == "cuda" else 64
+            chunks += [(ph, S, int(n), torch.tensor(idx[i:i + size], device=dev)) for i in range(0, len(idx), size)]
+
+    def evaluate(ph, S, n, idx, p):
+        rel = p[T["atoms"][idx, :n - 1]] - p[T["absorber"][idx]][:, None]
+        if box is not None:
+            rel = rel - box * torch.round(rel.detach() / box)
+        cchi, reff = _cchi(ph, torch.cat([torch.zeros_like(rel[:, :1]), rel], 1), T["ipots"][idx, :n])
+        return _chi(cchi, reff, S, qt, I["sigma2"])
+    with torch.no_grad():
+        for ph, S, n, idx in chunks:
+            chi = evaluate(ph, S, n, idx, pos)
+            seg.index_add_(0, T["segment"][idx], chi * T["deg"][idx, None])
+    if loss_grad is None:
+        return seg
+    g = loss_grad(seg)
+    p = pos.clone().requires_grad_()
+    for ph, S, n, idx in chunks:
+        chi = evaluate(ph, S, n, idx, p)
+        (chi * (T["deg"][idx, None] * g[T["segment"][idx]])).sum().backward()
+    return seg, p.grad
+
+
+def _r_factor(chi, data, nfft=2048, float32_grid=False):
+    """R-factor per row of chi against data in the window WINDOW."""
+    w, dev = WINDOW, chi.device
+    k = 0.05 * torch.arange(chi.shape[1], device=dev, dtype=torch.float64)
+    up, dn = ((k - (x - 0.5)).clamp(0, 1) for x in (w["kmin"], w["kmax"]))
+    f = k ** 2 * 0.25 * (1 - torch.cos(math.pi * up)) * (1 + torch.cos(math.pi * dn))
+    R = math.pi / (0.05 * nfft) * np.arange(nfft // 2, dtype=np.float32 if float32_grid else np.float64)
+    m = torch.tensor(np.nonzero((R >= w["rmin"]) & (R <= w["rmax"]))[0], device=dev, dtype=torch.float64)
+    tw = torch.exp(-2j * math.pi / nfft * (torch.arange(len(k), device=dev)[:, None] * m[None]))
+    D = ((chi - data) * f).to(tw.dtype) @ tw
+    B = (data * f).to(tw.dtype) @ tw
+    return (D.real ** 2 + D.imag ** 2).sum(-1) / (B.real ** 2 + B.imag ** 2).sum(-1)
+
+
+def exact(case, seed):
+    dev, kind = _dev(), case["kind"]
+    c = lambda a: torch.tensor(a, device=dev)       # noqa: E731
+    if kind == "stage":
+        rel, ipots, up = _walks(case, seed)
+        ph = _Phase(PHASES[case["edge"]], dev)
+        S, q = c(_grid(ph.kf, Q18, case["convention"])), c(Q18)
+        up = c(up) if case["precision"] == 64 else c(up).float().double()
+        out = []
+        for i in range(0, len(rel), 2048):
+            x = c(rel[i:i + 2048]).requires_grad_(case["grad"])
+            cchi, reff = _cchi(ph, x, c(ipots[i:i + 2048]))
+            chi = _chi(cchi, reff, S, q, None)
+            row = [torch.view_as_real(cchi.detach()), reff.detach(), chi.detach()]
+            out.append(row + ([torch.autograd.grad((chi * up[i:i + 2048]).sum(), x)[0]] if case["grad"] else []))
+        return [torch.cat(v) for v in zip(*out)]
+    if kind == "pairs":
+        return _pairs_exact(case, seed)
+    I = _inputs(case, seed)
+    if kind == "spectra":
+        en = Q18 ** 2 - case["e0"] * ETOK
+        q, tgt, out = np.sign(en) * np.sqrt(np.abs(en)), c(_target(1, Q18, seed)[0]), []
+
+        def spectra_grad(seg):
+            with torch.enable_grad():
+                s = seg.clone().requires_grad_()
+                chi = s / case["absorbers"]
+                mis = _r_factor(chi.mean(0)[None], tgt, float32_grid=True)[0]
+                out.extend([chi.detach(), mis.detach()])
+                return torch.autograd.grad(mis, s)[0]
+        grad = _list_exact(I, q, spectra_grad)[1]
+        return out + [grad]
+    q = I["q"]
+    if kind == "trajectory":
+        return _list_exact(I, q, None)
+    if not case.get("captured"):
+        up = c(_weights(I["nseg"], q, seed))
+        return list(_list_exact(I, q, lambda s: up))
+    tgt = c(_target(I["nseg"], q, seed))
+    if kind != "refine":
+        return list(_list_exact(I, q, lambda s: 2 * c(q ** 2) * (s - tgt)))
+    rf = []
+
+    def refine_grad(seg):
+        with torch.enable_grad():
+            s = seg.clone().requires_grad_()
+            r = _r_factor(s, tgt)
+            rf.append(r.detach())
+            return torch.autograd.grad(r.sum(), s)[0]
+    return list(_list_exact(I, q, refine_grad)) + rf
+
+
+def _pairs_exact(case, seed):
+    """Single scattering from linearly interpolated two-leg signals on the distance grid, and its gradient."""
+    dev = _dev()
+    pos, ipot, _, box, up = _pair_inputs(case, seed)
+    ph = _Phase(PHASES["K"], dev)
+    S, q = torch.tensor(_grid(ph.kf, Q18, "feff"), device=dev), torch.tensor(Q18, device=dev)
+    up, box = torch.tensor(up, device=dev), torch.tensor(box, device=dev)
+    nr = int(round((case["rmax"] - 1.5) / 0.002)) + 1
+    r = (1.5 + 0.002 * torch.arange(nr, device=dev, dtype=torch.float32)).double()
+    ip = torch.tensor(ipot, device=dev)
+    table = {}
+    for p in (1, 2):
+        xyz = torch.stack([torch.zeros_like(r), torch.zeros_like(r), r], -1)
+        xyz = torch.stack([torch.zeros_like(xyz), xyz], 1)
+        cchi, reff = _cchi(ph, xyz, torch.tensor([[0, p]], device=dev).expand(nr, 2))
+        table[p] = _chi(cchi, reff, S, q, None)
+    F, n = pos.shape[:2]
+    G = torch.stack([table[p] @ up for p in (1, 2)]) / (F * n)
+    hist = torch.zeros(2, nr, dtype=torch.float64, device=dev)
+    grads = []
+    for f in range(F):
+        x = torch.tensor(pos[f], device=dev)
+        v = x[None] - x[:, None]                            # neighbour j - absorber a
+        v -= box * torch.round(v / box)
+        d2 = (v ** 2).sum(-1)
+        a, j = torch.nonzero((d2 <= case["rmax"] ** 2) & (d2 > 1e-6), as_tuple=True)
+        d, v = torch.sqrt(d2[a, j]), v[a, j]
+        u = (d - 1.5) / 0.002
+        i0 = u.floor().clamp(0, nr - 2).long()
+        w = u - i0
+        inside = (w >= 0) & (w <= 1)
+        w = w.clamp(0, 1)
+        k = ip[j] - 1
+        hist.view(-1).index_add_(0, k * nr + i0, 1 - w).index_add_(0, k * nr + i0 + 1, w)
+        s = torch.where(inside, (G[k, i0 + 1] - G[k, i0]) / 0.002, torch.zeros_like(d)) / d
+        g = torch.zeros_like(x)
+        grads.append(g.index_add_(0, j, s[:, None] * v).index_add_(0, a, -s[:, None] * v))
+    chi = (hist[0] @ table[1] + hist[1] @ table[2]) / (F * n)
+    return [chi, torch.stack(grads)]
