@@ -1,6 +1,6 @@
 """What a user of this framework has it do, as timed cases: the path stage on explicit paths, on held path lists (eager
-calls with their gradient and captured steps), the whole-call forward models with path finder and misfit, and single scattering from pair
-tables.
+calls with their gradient and captured steps), the whole-call forward models with path finder and misfit, and single
+scattering from pair tables.
 
 listed() names the cases, draw(rng) gives more of the same ranges, prepare(case, seed) makes what a program holds
 before the call, run(state) is one pass through the public entry points, work(case) counts what the pass cannot do
@@ -441,7 +441,8 @@ def work(case):
         B, n, b = case["paths"], case["legs"], case["precision"] // 8
         fl = path_cmacs(T, np.full(B, n), ipots).sum() * FLOPS_PER_CMAC
         by = B * (n * 32 + 2 * T.E * b + b + nk * b)
-        return {"bytes": by + (B * (nk * b + n * 24) if case["grad"] else 0), "flops": fl * (3 if case["grad"] else 1)}
+        return {"bytes": by + (B * (nk * b + n * 24) if case["grad"] else 0),
+                "flops": float(fl * (3 if case["grad"] else 1))}
     if kind == "pairs":
         n = 2 * case["cells"] ** 3 if case["structure"] == "bcc" else 8 * case["nx"] * case["ny"] * case["nz"]
         nr, npot = int(round((case["rmax"] - 1.5) / 0.002)) + 1, NPOT["K"]
@@ -452,7 +453,7 @@ def work(case):
     fl, P, n, nseg, nk = _path_work(key)
     grad = kind != "trajectory"
     by = n * (48 if grad else 24) + P * 40 + nseg * nk * (16 if grad else 4)
-    return {"bytes": int(by), "flops": (3 if grad else 1) * fl}
+    return {"bytes": int(by), "flops": float((3 if grad else 1) * fl)}
 
 
 # ---------------------------------------------------------------------------------------------------- in 64 bits
