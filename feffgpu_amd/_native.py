@@ -165,6 +165,11 @@ def lib():
         L.fm_pair_histogram.argtypes = [_i32, _i32, _vp, _i32, _vp, _vp, _i32, ctypes.POINTER(FmPairGrid), _vp, _vp,
                                         _vp]
         L.fm_pair_histogram_grad.argtypes = [_i32, _i32, _vp, _vp, _i32, ctypes.POINTER(FmPairGrid), _vp, _vp, _vp]
+        L.fm_pair_chi_workspace_bytes.restype = _sz
+        L.fm_pair_chi_workspace_bytes.argtypes = [_i32, _i32, _i32]
+        L.fm_pair_chi.argtypes = [_i32, _P(_vp), _P(_i32), _i32, _i32, _i32, _vp, _i32, ctypes.c_double, _vp, _vp, _sz,
+                                  _vp]
+        L.fm_pair_chi_grad.argtypes = [_i32, _P(_vp), _P(_i32), _i32, _i32, _i32, _vp, ctypes.c_double, _vp, _vp]
         L.fm_set_lds_budget.restype = _i32
         L.fm_set_lds_budget.argtypes = [_i32, _i32]
         _lib = L

@@ -158,6 +158,14 @@ class PairTables:
         return _SingleScattering.apply(pos, self)
 
 
+def _table_args(T, pots, nr):
+    """The tables T of the potentials pots as fm_pair_chi takes them: (pointers, histogram rows, precision)."""
+    if any(t.dim() != 2 or t.shape[0] != nr or t.shape != T[0].shape for t in T):
+        raise ValueError("the tables must have one shape (nr, NK)")
+    return ((ctypes.c_void_p * len(T))(*[t.data_ptr() for t in T]), (ctypes.c_int32 * len(T))(*pots),
+            32 if T[0].dtype == torch.float32 else 64)
+
+
 class _SingleScattering(torch.autograd.Function):
     @staticmethod
     def forward(ctx, pos, pt):
@@ -172,7 +180,7 @@ class _SingleScattering(torch.autograd.Function):
         g = pt._grid()
         # configurations in chunks of at most _BIN_PAIRS ordered pairs (the fixed-point bins' capacity), summed in FP64
         per = max(1, (_BIN_PAIRS - 1) // max(1, n * (n - 1)))
-        h = torch.zeros(pt.npot, pt.nr, dtype=torch.float64, device=pos.device)
+        h = None
         hist = torch.empty(pt.npot, pt.nr, dtype=torch.int64, device=pos.device)
         for c0 in range(0, C, per):
             cc = min(per, C - c0)
@@ -180,25 +188,36 @@ class _SingleScattering(torch.autograd.Function):
             N.check(N.lib().fm_pair_histogram(cc, n, P[c0:c0 + cc].data_ptr(), 0, None, ip.data_ptr(), pt.npot,
                                               ctypes.byref(g), hist.data_ptr(), None, N.stream_of(pos.device)),
                     "fm_pair_histogram")
-            h += hist.double() / _ONE
+            if per < C:
+                h = hist.double() / _ONE if h is None else h + hist.double() / _ONE
+        # the tables in one type for the products: float32 as built, float64 if any was replaced by another type
         pots = sorted(pt.tables)
-        T = pt.table_stack(pots)                                   # (P, nr, NK) float64
-        chi = sum(torch.mv(T[i].t().contiguous(), h[p]) for i, p in enumerate(pots)) / (C * n)
-        ctx.save_for_backward(P, ip, T)
+        tt = torch.float32 if all(pt.tables[p].dtype == torch.float32 for p in pots) else torch.float64
+        T = [pt.tables[p].to(device=pos.device, dtype=tt).contiguous() for p in pots]
+        ptrs, rows, prec = _table_args(T, pots, pt.nr)
+        nk = T[0].shape[1]
+        L = N.lib()
+        ws = torch.empty(int(L.fm_pair_chi_workspace_bytes(len(T), pt.nr, nk)), dtype=torch.uint8, device=pos.device)
+        chi = torch.empty(nk, dtype=torch.float64, device=pos.device)
+        N.check(L.fm_pair_chi(len(T), ptrs, rows, prec, pt.nr, nk, (hist if h is None else h).data_ptr(),
+                              1 if h is None else 0, float(C * n), chi.data_ptr(), ws.data_ptr(), ws.numel(),
+                              N.stream_of(pos.device)), "fm_pair_chi")
+        ctx.save_for_backward(P, ip, *T)
         ctx.pt, ctx.pots, ctx.shape, ctx.dtype = pt, pots, (C, n), pos.dtype
         return chi.to(pos.dtype)
 
     @staticmethod
     def backward(ctx, gchi):
-        P, ip, T = ctx.saved_tensors
+        P, ip, *T = ctx.saved_tensors
         pt, (C, n) = ctx.pt, ctx.shape
         gbin = torch.zeros(pt.npot, pt.nr, dtype=torch.float64, device=P.device)
         gk = gchi.to(torch.float64).contiguous()
-        for i, p in enumerate(ctx.pots):
-            gbin[p] = torch.mv(T[i], gk) / (C * n)
+        ptrs, rows, prec = _table_args(T, ctx.pots, pt.nr)
+        N.check(N.lib().fm_pair_chi_grad(len(T), ptrs, rows, prec, pt.nr, T[0].shape[1], gk.data_ptr(), float(C * n),
+                                         gbin.data_ptr(), N.stream_of(P.device)), "fm_pair_chi_grad")
         grad = torch.empty(C, n, 3, dtype=torch.float64, device=P.device)
         g = pt._grid()
         N.check(N.lib().fm_pair_histogram_grad(C, n, P.data_ptr(), ip.data_ptr(), pt.npot, ctypes.byref(g),
-                                               gbin.contiguous().data_ptr(), grad.data_ptr(), N.stream_of(P.device)),
+                                               gbin.data_ptr(), grad.data_ptr(), N.stream_of(P.device)),
                 "fm_pair_histogram_grad")
         return grad.to(ctx.dtype), None

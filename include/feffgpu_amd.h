@@ -262,6 +262,19 @@ int fm_pair_histogram(int32_t nconf, int32_t natom, const double *pos, int32_t n
 int fm_pair_histogram_grad(int32_t nconf, int32_t natom, const double *pos, const int32_t *ipot, int32_t npot,
                            const fm_pair_grid *grid, const double *gbin, double *grad_pos, void *stream);
 
+/* Single scattering from the tables (forward.py:300-320): chi [nk] = sum over the npot potentials p and the bins i of
+ * hist[rows[p]][i] tables[p][i][:] / div. tables (host array of device pointers, each [nr][nk], float for precision 32,
+ * double for 64), rows (host) the histogram row of each; hist rows of nr: int64 in units of 2^-32 (fixed_point != 0) or
+ * double. Sums in FP64 in a fixed order; workspace of fm_pair_chi_workspace_bytes. */
+size_t fm_pair_chi_workspace_bytes(int32_t npot, int32_t nr, int32_t nk);
+int fm_pair_chi(int32_t npot, const void *const *tables, const int32_t *rows, int32_t precision, int32_t nr, int32_t nk,
+                const void *hist, int32_t fixed_point, double div, double *chi, void *workspace, size_t workspace_bytes,
+                void *stream);
+
+/* Its adjoint in the bins: gbin[rows[p]][i] = sum_k tables[p][i][k] gchi[k] / div for the npot rows (others untouched). */
+int fm_pair_chi_grad(int32_t npot, const void *const *tables, const int32_t *rows, int32_t precision, int32_t nr,
+                     int32_t nk, const double *gchi, double div, double *gbin, void *stream);
+
 /* ---------------------------------------------------------------- path finder (src/feffgpu/pathfinder.py) --------
  * FEFF's path finder for absorbers of one configuration, float32 as the reference: GPUPathFinder.enumerate
  * (pathfinder.py:211-279), importance (:72-94), degenerate_total (:135-158) and the importance filter (:266-279).

@@ -162,3 +162,57 @@ def test_edge_cases(tables):
     assert float(h.abs().sum()) == 0.0 and short == 0
     with pytest.raises(ValueError):
         pt.single_scattering(torch.zeros(1, 0, 3, device="cuda", dtype=torch.float64))
+
+
+@pytest.mark.parametrize("n", (1, 2, 63, 64, 129, 257, 700))
+@pytest.mark.parametrize("kind", ("cubic", "general", "oblique", "cluster", "far", "unwrapped"))
+def test_every_pair_once_whatever_the_tiles(tables, kind, n):
+    """The float32 candidate test drops no pair that counts: tile remainders, cells exactly two cutoffs wide and
+    narrower, an oblique cell, clusters far from the origin, coordinates many cells away. Every atom an absorber
+    (unordered pairs) gives the same integers as the list of all of them (ordered pairs), and both the oracle's."""
+    import ctypes
+
+    from feffgpu_amd import _native as N
+    pt, _, _ = tables
+    rng = np.random.default_rng(n)
+    L = 2 * pt.rmax
+    cell = {"cubic": L, "general": np.diag([L, 0.8 * L, 1.3 * L]), "cluster": None, "far": None, "unwrapped": L,
+            "oblique": np.array([[L, 0, 0], [0.45 * L, 0.9 * L, 0], [-0.3 * L, 0.4 * L, 0.8 * L]])}[kind]
+    pos = rng.uniform(0, L, (n, 3))
+    if kind == "far":
+        pos += np.array([3e4, -2e4, 5e3])
+    if kind == "unwrapped":
+        pos += L * rng.integers(-40, 40, (n, 3))
+    ipot = rng.integers(-1, pt.npot + 1, n)
+    P, ip = torch.tensor(pos, device="cuda"), torch.tensor(ipot, device="cuda")
+    h, short = pt.histogram(P, torch.arange(n, device="cuda"), ip, box=cell)
+    ref, rshort = oracle.pair_histogram(pos, np.arange(n), ipot, cell, pt.r0, pt.dr, pt.nr, pt.rmax, pt.npot)
+    assert short == rshort and float(np.abs(h.cpu().numpy() - ref).max()) < 2e-8 if n > 1 else short == rshort == 0
+    hist = torch.zeros(pt.npot, pt.nr, dtype=torch.int64, device="cuda")
+    g = pt._grid(cell)
+    N.check(N.lib().fm_pair_histogram(1, n, P.data_ptr(), 0, None, ip.to(torch.int32).contiguous().data_ptr(), pt.npot,
+                                      ctypes.byref(g), hist.data_ptr(), None, N.stream_of(pt.device)), "hist")
+    assert torch.equal(hist.double() / _ONE, h)
+
+
+def test_table_products(tables):
+    """chi and its bin gradient against torch's FP64 products of the same histogram, with tables of both types."""
+    pt, pos0, L = tables
+    rng = np.random.default_rng(3)
+    kept, ip0 = dict(pt.tables), getattr(pt, "ipot", None)
+    pt.ipot = torch.tensor(rng.integers(1, pt.npot, len(pos0)), device="cuda")
+    try:
+        for dt in (torch.float32, torch.float64):
+            pt.tables = {k: v.to(dt) for k, v in kept.items()}
+            pos = torch.tensor(W.displaced(pos0, 0.1, 8)[None], device="cuda", requires_grad=True)
+            chi = pt.single_scattering(pos)
+            h, _ = pt.histogram(pos[0].detach(), torch.arange(len(pos0), device="cuda"), pt.ipot, box=L)
+            ref = sum(pt.tables[p].double().t() @ h[p] for p in sorted(pt.tables)) / len(pos0)
+            assert float((chi.detach() - ref).abs().max() / ref.abs().max()) < 1e-12
+            assert torch.isfinite(torch.autograd.grad(chi.sum(), pos)[0]).all()
+    finally:
+        pt.tables = kept
+        if ip0 is None:
+            del pt.ipot
+        else:
+            pt.ipot = ip0
