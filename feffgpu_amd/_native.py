@@ -191,15 +191,16 @@ def ptr(t) -> int | None:
 
 
 def backward_workspace(precision: int, nlegmax: int, npath: int, device, E: int, max_slots: int = 4096,
-                       max_region_bytes: int = 1 << 30):
-    """A device buffer for the adjoints: band slots for the workgroups in flight (paths of 7-9 legs: a workgroup
-    takes one per band of its plan, at most 16), at most max_slots and no more than npath workgroups need; and, for
-    the fused adjoint (2-6 legs), a region of (4 nleg + 1) E complex per path of a launch plus one spare, for up to
-    npath paths and at most max_region_bytes (larger buckets run in chunks)."""
-    slots = max(16, min(int(max_slots), 16 * max(int(npath), 1)))
+                       max_region_bytes: int = 2 << 30):
+    """A device buffer for the adjoints: paths of 7-9 legs, band slots for the workgroups in flight (a workgroup takes
+    one per band of its plan, at most 16), at most max_slots and no more than npath workgroups need; paths of 2-6 legs,
+    for each of up to npath paths of a launch the chain's matrices, the scattering matrices and cchi of an adjoint whose
+    forward kept none, and a record, at most max_region_bytes (larger buckets run in chunks)."""
+    slots = max(16, min(int(max_slots), 16 * max(int(npath), 1))) if nlegmax > 6 else 16
     nbytes = lib().fm_backward_workspace_bytes(int(precision), int(nlegmax), slots)
-    per = (4 * min(int(nlegmax), 6) + 1) * int(E) * (8 if precision == 32 else 16)
-    nbytes = max(nbytes, min((int(npath) + 1) * per, int(max_region_bytes)))
+    n, ec = min(int(nlegmax), 6), 8 if precision == 32 else 16
+    per = (40 * (n - 1) + 1) * (int(E) + 3) * ec + 8 * (10 * n + 3)
+    nbytes = max(nbytes, min((int(npath) + 32) * per, int(max_region_bytes)))
     return torch.empty(max(nbytes, 1), dtype=torch.uint8, device=device)
 
 

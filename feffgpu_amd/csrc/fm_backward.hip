@@ -24,6 +24,8 @@
 #include <type_traits>
 
 #include "fm_device.h"
+#include "fm_grad.h"
+#include "fm_internal.h"
 #include "fm_path.h"
 
 using namespace fm;
@@ -183,27 +185,6 @@ __device__ __forceinline__ void fblock_bwd(const cx<T> (&K)[FM_NREP], cx<T> ck, 
 // with buffer instructions. The slice's descriptor is wave-uniform (scalar registers), the lane enters as one
 // 32-bit offset and the element as a scalar offset, so no 64-bit address is formed per element. Accesses outside
 // the slice read 0 and write nothing.
-constexpr int FM_RSRC_WORD3 = 0x00020000;   // buffer descriptor word 3 on gfx9: 32-bit data format, no swizzle
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t slice_rsrc(unsigned char *p, size_t bytes) {
-    return __builtin_amdgcn_make_buffer_rsrc(p, (short)0, (int)bytes, FM_RSRC_WORD3);
-}
-template <class E>
-__device__ __forceinline__ void buf_st(__amdgpu_buffer_rsrc_t rs, uint32_t vo, int so, const E &v) {
-    if constexpr (sizeof(E) == 4) {
-        unsigned x;
-        __builtin_memcpy(&x, &v, 4);
-        __builtin_amdgcn_raw_buffer_store_b32(x, rs, vo, so, 0);
-    } else if constexpr (sizeof(E) == 8) {
-        __attribute__((ext_vector_type(2))) unsigned x;
-        __builtin_memcpy(&x, &v, 8);
-        __builtin_amdgcn_raw_buffer_store_b64(x, rs, vo, so, 0);
-    } else {
-        static_assert(sizeof(E) == 16, "element of 4, 8 or 16 bytes");
-        __attribute__((ext_vector_type(4))) unsigned x;
-        __builtin_memcpy(&x, &v, 16);
-        __builtin_amdgcn_raw_buffer_store_b128(x, rs, vo, so, 0);
-    }
-}
 template <class E> struct LaneArray {
     __amdgpu_buffer_rsrc_t rs;
     uint32_t lo;           // lane * sizeof(E)
@@ -559,120 +540,7 @@ __device__ __forceinline__ void pass_B(const fm_edge &ed, const PathLDS &g, cons
     }
 }
 
-// ------------------------------------------------------------------------------------------------ fused adjoint
-// The adjoint of paths of NL legs in one sweep per energy, with nothing of the amplitude leaving the registers.
-// ptrac is a polynomial in the entries of the scattering matrices, so for every real parameter theta of the
-// geometry (leg lengths, angles, eta) the sweep forms the complex derivative D_theta = d ptrac / d theta without
-// the upstream gradient; the loss gradient is Re(pbc D_theta) with pbc = conj(dL/dptrac), applied once the
-// fine-grid adjoint of the whole path is known. Per energy: the F_s representatives of every scatterer (kept),
-// the termination with its tangents against Pre_n = F_{n-1} ... F_1, then s = n-1 .. 1: K_s from Pre_s (rebuilt
-// from the kept F) and U_s = T F_{n-1} ... F_{s+1}, the eta derivative, U_{s-1}, and the tangent stream of F_s.
-
-// Bit 2 aa + bb set: some representative of an NR x NC block has Hankel columns (aa + 1, bb + 1).
-template <int SET, int NR, int NC>
-__host__ __device__ constexpr unsigned group_mask() {
-    constexpr PairDef PD = pairdef(SET);
-    unsigned m = 0;
-    for (int k = 0; k < FM_NREP; ++k)
-        if (PD.ri[k] < NR && PD.rj[k] < NC) m |= 1u << (2 * (PD.a[k] - 1) + PD.b[k] - 1);
-    return m;
-}
-
-// One partial-wave row of a block's tangents contracted with K, accumulated as complex derivatives. y, yd: the
-// gamtl leg's factors and their tangents without the row's t-matrix factor t, which scales the row's three sums once.
-template <class T, int SET, int NR, int NC, class WRow>
-__device__ __forceinline__ void bwd_row_c(const cx<T> (&K)[FM_NREP], const cx<T> (&xa)[3], const cx<T> (&xd)[3],
-                                          const cx<T> (&y)[2], const cx<T> (&yd)[2], cx<T> t, const WRow &w,
-                                          const WRow &wd, cx<T> &dX, cx<T> &dY, cx<T> &dB) {
-    constexpr PairDef PD = pairdef(SET);
-    constexpr unsigned used = group_mask<SET, NR, NC>();
-    const cx<T> zero = mk<T>(T(0), T(0));
-    cx<T> Q[3][2], Qd[3][2];
-#pragma unroll
-    for (int aa = 0; aa < 3; ++aa) Q[aa][0] = Q[aa][1] = Qd[aa][0] = Qd[aa][1] = zero;
-#pragma unroll
-    for (int k = 0; k < FM_NREP; ++k)
-        if (PD.ri[k] < NR && PD.rj[k] < NC) {
-            const int aa = PD.a[k] - 1, bb = PD.b[k] - 1;
-            rfma(Q[aa][bb], K[k], w[k]);
-            rfma(Qd[aa][bb], K[k], wd[k]);
-        }
-    // dB: sum Qd[aa][bb] xa[aa] y[bb]; dY: sum Q[aa][bb] xa[aa] yd[bb]; dX: sum Q[aa][bb] xd[aa] y[bb]
-    cx<T> sB = zero, sY = zero, sX = zero;
-#pragma unroll
-    for (int bb = 0; bb < 2; ++bb) {
-        if (!((used >> bb) & 0x15u)) continue;
-        cx<T> rd = zero, r = zero, v = zero;
-#pragma unroll
-        for (int aa = 0; aa < 3; ++aa)
-            if ((used >> (2 * aa + bb)) & 1u) {
-                cfma4(rd, Qd[aa][bb], xa[aa]);
-                cfma4(r, Q[aa][bb], xa[aa]);
-                cfma4(v, Q[aa][bb], xd[aa]);
-            }
-        cfma4(sB, y[bb], rd);
-        cfma4(sY, yd[bb], r);
-        cfma4(sX, y[bb], v);
-    }
-    cfma4(dB, t, sB);
-    cfma4(dY, t, sY);
-    cfma4(dX, t, sX);
-}
-
-// The tangent stream of one scattering matrix (rows il = 1..ilx, t-matrix two rows ahead), complex derivatives.
-template <class T, int SET, int NR, int NC>
-__device__ __forceinline__ void fblock_bwd_c(const cx<T> (&K)[FM_NREP], cx<T> ck, T rX, T rY, int ilx,
-                                             const T *__restrict__ Wl, const T *__restrict__ Wdl,
-                                             const T *__restrict__ tl, int tlstride, cx<T> t1, cx<T> t2, cx<T> &dX,
-                                             cx<T> &dY, cx<T> &dB) {
-    dX = dY = dB = mk<T>(T(0), T(0));
-    Hank3T<T> X;
-    Hank2T<T> Y;
-    X.init(minus_i_over(ck * rX), rX);
-    Y.init(minus_i_over(ck * rY), rY);
-    cx<T> xa[3], xd[3], ya[2], yd[2];
-    // the t-matrix two rows ahead (rows past ilx repeat row ilx, which stays in the table); rows 1 and min(2, ilx)
-    // come from the caller
-    cx<T> t = t1;
-    cx<T> tn = t2;
-    // rows 1..4 unrolled (their seeds are explicit per row); a lane whose energy has fewer rows runs them with the
-    // t-matrix factor zero, which adds nothing
-#pragma unroll
-    for (int r = 1; r <= 4; ++r) {
-        X.seed_row(r, xa, xd);
-        if (r < 4) Y.seed_row(r, ya, yd); else Y.step(r, ya, yd);
-        const size_t rn = (size_t)(r + 2 < ilx ? r + 2 : ilx) * tlstride;
-        const cx<T> tnn = mk<T>(tl[rn], tl[rn + 1]);
-        // rows past ilx read the table's row ilx (inside the table, finite) and add zero
-        const cx<T> tr = r <= ilx ? t : mk<T>(T(0), T(0));
-        const size_t rw = (size_t)(r <= ilx ? r : ilx) * FM_NREP;
-        bwd_row_c<T, SET, NR, NC>(K, xa, xd, ya, yd, tr, Wl + rw, Wdl + rw, dX, dY, dB);
-        t = tn;
-        tn = tnn;
-    }
-    // as in fblock: the row's table values read before the recursion steps that hide them, two rows per iteration
-    auto row = [&](int r) {
-        T wv[FM_NREP], wdv[FM_NREP];
-        load_wrow<T, SET, NR, NC>(wv, Wl + (size_t)r * FM_NREP);
-        load_wrow<T, SET, NR, NC>(wdv, Wdl + (size_t)r * FM_NREP);
-        __builtin_amdgcn_sched_barrier(0);
-        X.step(r, xa, xd);
-        Y.step(r, ya, yd);
-        const size_t rn = (size_t)(r + 2 < ilx ? r + 2 : ilx) * tlstride;
-        const cx<T> tnn = mk<T>(tl[rn], tl[rn + 1]);
-        bwd_row_c<T, SET, NR, NC>(K, xa, xd, ya, yd, t, wv, wdv, dX, dY, dB);
-        t = tn;
-        tn = tnn;
-    };
-    int r = 5;
-#pragma unroll 1
-    for (; r < ilx; r += 2) {
-        row(r);
-        row(r + 1);
-    }
-    if (r == ilx) row(r);
-}
-
+// ------------------------------------------------------------------------------------------------ single scattering
 // Complex derivative slots of a lane, (kind, leg j) -> slot kind nleg + j - 1, in the workspace region of the lane's
 // path: slot s of the lane's energy at byte lo + s sbytes (lo: the lane's (path, energy) offset in slot 0, sbytes: E
 // complex).
@@ -682,280 +550,6 @@ template <class T> struct DSlots {
     int sbytes, nleg;
     __device__ __forceinline__ void put(int kind, int j, cx<T> x) const { buf_st(rs, lo, (kind * nleg + j - 1) * sbytes, x); }
 };
-
-// F(i, j) of a block from its representatives, with the row phase: ph[i] sg Ft[idx[i][j]]
-template <class T, int SET>
-__device__ __forceinline__ cx<T> fent(const cx<T> (&Ft)[FM_NREP], const cx<T> (&ph)[6], int i, int j) {
-    constexpr PairDef PD = pairdef(SET);
-    return ph[i] * Ft[PD.idx[i][j]] * T(PD.sg[i][j]);
-}
-
-// Pre_S = F_{S-1} ... F_1 (L x L0, with the row phases) from the kept representatives; S >= 2.
-template <class T, int SET, int NL, int S>
-__device__ __forceinline__ void prefix(const PathLDS &g, const cx<T> (&F)[NL - 1][FM_NREP],
-                                       cx<T> (&P)[lamdef(SET).L][lamdef(SET).L0]) {
-    constexpr int L = lamdef(SET).L, L0 = lamdef(SET).L0;
-    cx<T> ph[6];
-    row_phases<T, SET>(ph, g, 2);
-#pragma unroll
-    for (int i = 0; i < L; ++i)
-#pragma unroll
-        for (int b = 0; b < L0; ++b) P[i][b] = fent<T, SET>(F[0], ph, i, b);
-#pragma unroll
-    for (int t = 2; t < S; ++t) {   // Pre_{t+1} = F_t Pre_t
-        row_phases<T, SET>(ph, g, t + 1);
-#pragma unroll
-        for (int b = 0; b < L0; ++b) {
-            cx<T> col[L];
-#pragma unroll
-            for (int j = 0; j < L; ++j) col[j] = P[j][b];
-#pragma unroll
-            for (int i = 0; i < L; ++i) {
-                cx<T> acc = mk<T>(T(0), T(0));
-#pragma unroll
-                for (int j = 0; j < L; ++j) cfma4(acc, fent<T, SET>(F[t - 1], ph, i, j), col[j]);
-                P[i][b] = acc;
-            }
-        }
-    }
-}
-
-// What a chain step needs of its scatterer S at the lane's energy: the partial waves ilx, the scatterer's t-matrix
-// column and its rows 1 and min(2, ilx) (row 2 read whole from min(2, L1), used only when ilx >= 2).
-template <class T> struct ScatIn {
-    int ilx;
-    const T *tl;
-    cx<T> t1, t2;
-};
-template <class T>
-__device__ __forceinline__ ScatIn<T> scat_in(const fm_edge &ed, const PathLDS &g, int ltab, int ee, int S) {
-    const int E = ed.E, ip = g.ipot[S];
-    const T *tl = TL<T>::tl(ed) + ((size_t)ip * ltab) * (2 * E) + 2 * ee;
-    const size_t r2 = (size_t)(ed.L1 < 2 ? ed.L1 : 2) * (2 * E);
-    return ScatIn<T>{ed.lmax[(size_t)ip * E + ee] + 1, tl, mk<T>(tl[2 * E], tl[2 * E + 1]), mk<T>(tl[r2], tl[r2 + 1])};
-}
-// Whether the sweep reads every scatterer's ScatIn when the energy starts (their loads in flight together, hidden by
-// Pre_n) or at its chain step: early where the registers hold them without more spills (measured: K edges up to 4
-// legs, L/M edges 3 legs).
-template <int SET, int NL> constexpr bool scat_early() { return NL <= (SET == 0 ? 4 : 3); }
-
-// One chain step of the fused sweep (scatterer S; NR x NC block): K and the eta derivative from Pre_S and U, then
-// U <- U F_S (unless S = 1), then the tangent stream of F_S.
-template <class T, int SET, int NL, int S>
-__device__ __forceinline__ void fused_step(const fm_edge &ed, const PathLDS &g, const T *W, const T *Wd, int ltab, int ee,
-                                           cx<T> ck, const ScatIn<T> (&sc)[NL - 1], const cx<T> (&F)[NL - 1][FM_NREP],
-                                           cx<T> (&U)[lamdef(SET).L0][lamdef(SET).L], DSlots<T> ds) {
-    constexpr LamDef D = lamdef(SET);
-    constexpr PairDef PD = pairdef(SET);
-    constexpr int L = D.L, L0 = D.L0;
-    constexpr int NR = S == NL - 1 ? L0 : L, NC = S == 1 ? L0 : L;
-    const int E = ed.E;
-    cx<T> ph[6];
-    row_phases<T, SET>(ph, g, S + 1);
-    cx<T> K[FM_NREP];
-    {
-        cx<T> P[L][L0];
-        if constexpr (S >= 2) prefix<T, SET, NL, S>(g, F, P);
-#pragma unroll
-        for (int k = 0; k < FM_NREP; ++k) K[k] = mk<T>(T(0), T(0));
-        // K from Pre_S and U; the eta_{S+1} derivative -i sum_{l1,l2} M[l1] h(l1, l2) F_S(l1, l2) on the way
-        cx<T> de = mk<T>(T(0), T(0));
-#pragma unroll
-        for (int l2 = 0; l2 < NC; ++l2) {
-#pragma unroll
-            for (int l1 = 0; l1 < NR; ++l1) {
-                cx<T> m = mk<T>(T(0), T(0));
-                if constexpr (S >= 2) {
-#pragma unroll
-                    for (int a = 0; a < L0; ++a) cfma4(m, P[l2][a], U[a][l1]);
-                } else {
-                    m = U[l2][l1];
-                }
-                const cx<T> h = m * ph[l1];
-                if (PD.sg[l1][l2] > 0) K[PD.idx[l1][l2]] = K[PD.idx[l1][l2]] + h;
-                else K[PD.idx[l1][l2]] = K[PD.idx[l1][l2]] - h;
-                if (D.M[l1] != 0) cfma4(de, h * T(PD.sg[l1][l2] * D.M[l1]), F[S - 1][PD.idx[l1][l2]]);
-            }
-        }
-        ds.put(GK_H, S + 1, mk<T>(de.i, -de.r));
-        if constexpr (S > 1) {
-#pragma unroll
-            for (int a = 0; a < L0; ++a) {
-                cx<T> row[6];
-#pragma unroll
-                for (int i = 0; i < 6; ++i) row[i] = (i < NR) ? U[a][i] * ph[i] : mk<T>(T(0), T(0));
-#pragma unroll
-                for (int j = 0; j < L; ++j) {
-                    cx<T> v = mk<T>(T(0), T(0));
-                    if (j < NC) {
-#pragma unroll
-                        for (int i = 0; i < NR; ++i) {
-                            const cx<T> f = F[S - 1][PD.idx[i][j]];
-                            if (PD.sg[i][j] > 0) cfma4(v, row[i], f); else cfma4(v, row[i], mk<T>(-f.r, -f.i));
-                        }
-                    }
-                    U[a][j] = v;
-                }
-            }
-        }
-    }
-    ScatIn<T> si;
-    if constexpr (scat_early<SET, NL>()) si = sc[S - 1];
-    else si = scat_in<T>(ed, g, ltab, ee, S);
-    cx<T> dX, dY, dB;
-    fblock_bwd_c<T, SET, NR, NC>(K, ck, (T)g.r[S + 1], (T)g.r[S], si.ilx, W + (size_t)(S - 1) * ltab * FM_NREP,
-                                 Wd + (size_t)(S - 1) * ltab * FM_NREP, si.tl, 2 * E, si.t1,
-                                 si.ilx >= 2 ? si.t2 : si.t1, dX, dY, dB);
-    ds.put(GK_X, S + 1, dX);
-    ds.put(GK_Y, S, dY);
-    ds.put(GK_B, S, dB);
-}
-
-template <class T, int SET, int NL, int S>
-__device__ __forceinline__ void fused_chain(const fm_edge &ed, const PathLDS &g, const T *W, const T *Wd, int ltab, int ee,
-                                            cx<T> ck, const ScatIn<T> (&sc)[NL - 1], const cx<T> (&F)[NL - 1][FM_NREP],
-                                            cx<T> (&U)[lamdef(SET).L0][lamdef(SET).L], DSlots<T> ds) {
-    fused_step<T, SET, NL, S>(ed, g, W, Wd, ltab, ee, ck, sc, F, U, ds);
-    if constexpr (S > 1) fused_chain<T, SET, NL, S - 1>(ed, g, W, Wd, ltab, ee, ck, sc, F, U, ds);
-}
-
-template <class T, int SET, int NL, int S>
-__device__ __forceinline__ void fused_fblocks(const fm_edge &ed, const PathLDS &g, const T *W, int ltab, int ee,
-                                              cx<T> (&F)[NL - 1][FM_NREP]) {
-    constexpr int L = lamdef(SET).L, L0 = lamdef(SET).L0;
-    const int E = ed.E;
-    const cx<T> ck = mk<T>((T)ed.ck[2 * ee], (T)ed.ck[2 * ee + 1]);
-    const int ip = g.ipot[S];
-    const int ilx = ed.lmax[(size_t)ip * E + ee] + 1;
-    const T *tl = TL<T>::tl(ed) + ((size_t)ip * ltab) * (2 * E) + 2 * ee;
-    const T *Wl = W + (size_t)(S - 1) * ltab * FM_NREP;
-    if constexpr (S == 1) fblock<T, SET, L, L0, true>(F[0], ck, (T)g.r[2], (T)g.r[1], ilx, Wl, tl, 2 * E);
-    else if constexpr (S == NL - 1) fblock<T, SET, L0, L, true>(F[S - 1], ck, (T)g.r[S + 1], (T)g.r[S], ilx, Wl, tl, 2 * E);
-    else fblock<T, SET, L, L, true>(F[S - 1], ck, (T)g.r[S + 1], (T)g.r[S], ilx, Wl, tl, 2 * E);
-    if constexpr (S < NL - 1) fused_fblocks<T, SET, NL, S + 1>(ed, g, W, ltab, ee, F);
-}
-
-// The kept matrices of scatterers S..NL-1 from the lane's rows (the first scatterer's block is L x L0, the last's
-// L0 x L, the others L x L).
-template <class T, int SET, int NL, int S>
-__device__ __forceinline__ void keep_loads(const T *kp, int E, cx<T> (&F)[NL - 1][FM_NREP]) {
-    constexpr int L = lamdef(SET).L, L0 = lamdef(SET).L0;
-    const T *b = kp + (size_t)2 * E * keep_off<SET>(NL, S);
-    if constexpr (S == 1) keep_load<T, SET, L, L0>(b, E, F[S - 1]);
-    else if constexpr (S == NL - 1) keep_load<T, SET, L0, L>(b, E, F[S - 1]);
-    else keep_load<T, SET, L, L>(b, E, F[S - 1]);
-    if constexpr (S < NL - 1) keep_loads<T, SET, NL, S + 1>(kp, E, F);
-}
-
-// The fused sweep at energy ee from the scattering matrices F of every scatterer (kept by the forward or rebuilt):
-// returns cchi and stores the complex derivatives of ptrac in ds.
-template <class T, int SET, int NL>
-__device__ __forceinline__ cx<T> fused_energy(const fm_edge &ed, const PathLDS &g, const T *W, const T *Wd, int ltab,
-                                              int ee, DSlots<T> ds, const cx<T> (&F)[NL - 1][FM_NREP]) {
-    constexpr LamDef D = lamdef(SET);
-    constexpr PairDef PD = pairdef(SET);
-    constexpr int L = D.L, L0 = D.L0;
-    const int E = ed.E;
-    // read ahead of Pre_n, whose work hides their latency: the termination's channel weights of rows 1..4 (a row
-    // without a channel reads channel 0's and does not use it), ck, and (scat_early) every scatterer's ScatIn
-    const cx<T> ck = mk<T>((T)ed.ck[2 * ee], (T)ed.ck[2 * ee + 1]);
-    ScatIn<T> sc[NL - 1];
-    if constexpr (scat_early<SET, NL>()) {
-#pragma unroll
-        for (int S = 1; S < NL; ++S) sc[S - 1] = scat_in<T>(ed, g, ltab, ee, S);
-    }
-    const T *chw = TL<T>::chw(ed);
-    int chan[4];
-    cx<T> wraw[4];
-#pragma unroll
-    for (int r = 1; r <= 4; ++r) {
-        int c = -1;
-        for (int q = 0; q < ed.nchan; ++q)
-            if (ed.chan_il[q] == r) c = q;
-        chan[r - 1] = c;
-        const size_t o = ((size_t)(c >= 0 ? c : 0) * E + ee) * 2;
-        wraw[r - 1] = mk<T>(chw[o], chw[o + 1]);
-    }
-    // Pre_n (L0 x L0)
-    cx<T> Pn[L0][L0];
-    {
-        cx<T> P[L][L0];
-        prefix<T, SET, NL, NL - 1>(g, F, P);
-        cx<T> ph[6];
-        row_phases<T, SET>(ph, g, NL);
-#pragma unroll
-        for (int i = 0; i < L0; ++i)
-#pragma unroll
-            for (int b = 0; b < L0; ++b) {
-                cx<T> acc = mk<T>(T(0), T(0));
-#pragma unroll
-                for (int j = 0; j < L; ++j) cfma4(acc, fent<T, SET>(F[NL - 2], ph, i, j), P[j][b]);
-                Pn[i][b] = acc;
-            }
-    }
-    // termination: T with its tangents against K_T[a][b] = Pn[b][a] ph1[a]
-    cx<T> U[L0][L];
-    cx<T> ptrac = mk<T>(T(0), T(0));
-    {
-        cx<T> ph[6];
-        row_phases<T, SET>(ph, g, 1);
-        cx<T> K[FM_NREP];
-#pragma unroll
-        for (int k = 0; k < FM_NREP; ++k) K[k] = mk<T>(T(0), T(0));
-#pragma unroll
-        for (int a = 0; a < L0; ++a)
-#pragma unroll
-            for (int b = 0; b < L0; ++b) {
-                const cx<T> h = Pn[b][a] * ph[a];
-                if (PD.sg[a][b] > 0) K[PD.idx[a][b]] = K[PD.idx[a][b]] + h;
-                else K[PD.idx[a][b]] = K[PD.idx[a][b]] - h;
-            }
-        const int *lm = ed.lmax + ee;
-        const int lx1 = max(lm[(size_t)g.ipot[0] * E], lm[(size_t)g.ipot[1] * E]) + 1;
-        const int lxn = max(lm[(size_t)g.ipot[NL - 1] * E], lm[(size_t)g.ipot[NL] * E]) + 1;
-        Hank3T<T> X;
-        Hank2T<T> Y;
-        X.init(minus_i_over(ck * (T)g.r[1]), (T)g.r[1]);
-        Y.init(minus_i_over(ck * (T)g.r[NL]), (T)g.r[NL]);
-        cx<T> Tt[FM_NREP];
-#pragma unroll
-        for (int k = 0; k < FM_NREP; ++k) Tt[k] = mk<T>(T(0), T(0));
-        const T *Wn = W + (size_t)(NL - 1) * ltab * FM_NREP;
-        const T *Wdn = Wd + (size_t)(NL - 1) * ltab * FM_NREP;
-        cx<T> dX = mk<T>(T(0), T(0)), dY = dX, dB = dX;
-        cx<T> xa[3], xd[3], ya[2], yd[2];
-#pragma unroll
-        for (int r = 1; r <= 4; ++r) {
-            X.seed_row(r, xa, xd, r <= lx1);
-            if (r < 4) Y.seed_row(r, ya, yd, r <= lxn); else Y.step(r, ya, yd, r <= lxn);
-            if (chan[r - 1] >= 0) {
-                const cx<T> w = wraw[r - 1] * T(2 * r - 1);
-                accum_row<T, SET, L0, L0>(Tt, xa, ya[0] * w, ya[1] * w, Wn + (size_t)r * FM_NREP);
-                bwd_row_c<T, SET, L0, L0>(K, xa, xd, ya, yd, w, Wn + (size_t)r * FM_NREP, Wdn + (size_t)r * FM_NREP,
-                                          dX, dY, dB);
-            }
-        }
-        ds.put(GK_X, 1, dX);
-        ds.put(GK_Y, NL, dY);
-        ds.put(GK_B, NL, dB);
-        cx<T> de = mk<T>(T(0), T(0));
-#pragma unroll
-        for (int a = 0; a < L0; ++a)
-#pragma unroll
-            for (int b = 0; b < L; ++b) {
-                const cx<T> t = (b < L0) ? ph[a] * Tt[PD.idx[a][b]] * T(PD.sg[a][b]) : mk<T>(T(0), T(0));
-                U[a][b] = t;
-                if (b < L0) {
-                    const cx<T> tp = t * Pn[b][a];
-                    ptrac = ptrac + tp;
-                    if (D.M[a] != 0) rfma(de, tp, T(D.M[a]));
-                }
-            }
-        ds.put(GK_H, 1, mk<T>(de.i, -de.r));
-    }
-    fused_chain<T, SET, NL, NL - 1>(ed, g, W, Wd, ltab, ee, ck, sc, F, U, ds);
-    return ptrac * cfac_at<T>(ed, g, ee, NL);
-}
 
 // The geometry adjoint of one path (one wavefront): for direction lane < ndir (atom lane / 3, plus 1 for a path list
 // whose absorber is atom 0; component lane % 3), the sum over the legs J of gp . d(r_J, beta_J, gamma_J, alpha_{J+1})
@@ -992,172 +586,6 @@ __device__ __forceinline__ double geometry_adjoint(const PathLDS &g, int n, int 
         for (int J = 0; J < n; ++J) acc += scr[lane * n + J];
     wave_sync();
     return acc / FM_BOHR;
-}
-
-// deterministic wave sum (butterfly)
-__device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, FM_WAVE);
-    return v;
-}
-
-// amp / unwrapped phase of cc[0..E) into amp[], ang[] (the forward epilogue's first half)
-template <class T>
-__device__ __forceinline__ void amp_phase(int E, const cx<T> *cc, T *amp, double *ang) {
-    const int lane = lane_id();
-    for (int e = lane; e < E; e += FM_WAVE) {
-        amp[e] = (T)sqrt((double)cc[e].r * cc[e].r + (double)cc[e].i * cc[e].i + 1e-30);
-        ang[e] = (double)atan2(cc[e].i, cc[e].r);
-    }
-    wave_sync();
-    const double a0 = ang[0];
-    double dl[FM_MAX_ECHUNK];
-#pragma unroll
-    for (int c = 0; c < FM_MAX_ECHUNK; ++c) {
-        const int e = c * FM_WAVE + lane;
-        double d = 0.0;
-        if (e < E && e > 0) {
-            d = ang[e] - ang[e - 1];
-            d -= FM_TWO_PI * rint(d / FM_TWO_PI);
-        }
-        dl[c] = d;
-    }
-    wave_sync();
-    double carry = 0.0;
-#pragma unroll
-    for (int c = 0; c < FM_MAX_ECHUNK; ++c) {
-        if (c * FM_WAVE >= E) break;
-        const int e = c * FM_WAVE + lane;
-        const double s = wave_scan_add(dl[c]) + carry;
-        carry = __shfl(s, FM_WAVE - 1, FM_WAVE);
-        if (e < E) ang[e] = a0 + s;
-    }
-    wave_sync();
-}
-
-// Adjoint of the fine grid of one path (one wave): chi(q) = A(q) sin(Phi(q) + 2 q reff) exp(-2 sigma2 q^2), A and
-// Phi linear in amp[] and the unwrapped ang[]. From dL/dchi(q) = gup_scale gup_d[q] + gup_p[q] to dL/dcchi per
-// energy: each energy gathers the q points that interpolate from it (qorder / qstart runs, in a fixed order).
-// With qs (3 nk doubles of LDS), dL/dA(q), dL/dPhi(q) and the fraction are first evaluated once per q point with
-// the lanes over the points (their loads independent), then gathered from LDS; without it, each energy evaluates
-// them where it uses them. Returns dL/dreff (A), wave-summed.
-template <class T>
-__device__ __forceinline__ double fine_grid_adjoint(int E, const int32_t *jq, const double *fq, const double *q, const int32_t *qorder,
-                                    const int32_t *qstart, double reff_A, double sigma2, const double *gup_d,
-                                    double gup_scale, const T *gup_p, const cx<T> *cc, const T *amp, const double *ang,
-                                    cx<T> *cb, int nk = 0, double *qs = nullptr, const double *S = nullptr,
-                                    int sstride = 0) {
-    const int lane = lane_id();
-    // dL/dA and dL/dPhi at q point i from its interpolation (j, f), q and the upstream gradient gu
-    auto eval = [&](int j, double f, double qi, double gu, double &gA, double &gP) {
-        const double A = (1.0 - f) * (double)amp[j] + f * (double)amp[j + 1];
-        double ph = (1.0 - f) * ang[j] + f * ang[j + 1] + 2.0 * qi * reff_A;
-        ph -= FM_TWO_PI * rint(ph / FM_TWO_PI);
-        if (sigma2 != 0.0) gu *= exp(-2.0 * sigma2 * qi * qi);
-        T sn, cs;
-        if constexpr (sizeof(T) == 4) sincosf((float)ph, &sn, &cs); else sincos(ph, &sn, &cs);
-        gA = (double)(T)(gu * (double)sn);
-        gP = (double)(T)(gu * A * (double)cs);
-    };
-    auto gup = [&](int i) -> double {
-        double gu = 0.0;
-        if (gup_d) gu += gup_scale * gup_d[i];
-        if (gup_p) gu += (double)gup_p[i];
-        return gu;
-    };
-    auto adj = [&](int i, double &gA, double &gP) { eval(jq[i], fq[i], q[i], gup(i), gA, gP); };
-    double rb = 0.0;
-    // dL/dcchi at energy e from dL/dA and dL/dPhi there (through amp = |cchi| and the phase)
-    auto finish = [&](int e, double ab, double pb) {
-        const double cr = (double)cc[e].r, ci = (double)cc[e].i;
-        const double c2 = cr * cr + ci * ci, a = (double)amp[e];
-        cx<T> v = mk<T>(T(0), T(0));
-        if (c2 > 0.0) v = mk<T>((T)(ab * cr / a - pb * ci / c2), (T)(ab * ci / a + pb * cr / c2));
-        cb[e] = v;
-    };
-    // staging: dL/dA and dL/dPhi per q point (values already rounded to T, so stored as T), then the fractions
-    T *const sA = qs ? reinterpret_cast<T *>(qs) : nullptr;
-    T *const sP = qs ? sA + nk : nullptr;
-    double *const sF = qs ? reinterpret_cast<double *>(sP + nk) : nullptr;
-    if (S) {   // dense interpolation (qs required): dL/dA, dL/dPhi per q point, then S^T per energy
-        for (int i = lane; i < nk; i += FM_WAVE) {
-            const double *Si = S + (size_t)i * sstride;
-            double sa = 0.0, sp = 0.0;
-            for (int e = 0; e < E; ++e) {
-                sa += Si[e] * (double)amp[e];
-                sp += Si[e] * ang[e];
-            }
-            double ph = sp + 2.0 * q[i] * reff_A;
-            ph -= FM_TWO_PI * rint(ph / FM_TWO_PI);
-            double gu = gup(i);
-            if (sigma2 != 0.0) gu *= exp(-2.0 * sigma2 * q[i] * q[i]);
-            T sn, cs;
-            if constexpr (sizeof(T) == 4) sincosf((float)ph, &sn, &cs); else sincos(ph, &sn, &cs);
-            const double gP = (double)(T)(gu * sa * (double)cs);
-            sA[i] = (T)(gu * (double)sn);
-            sP[i] = (T)gP;
-            rb += 2.0 * q[i] * gP;
-        }
-        wave_sync();
-        for (int e = lane; e < E; e += FM_WAVE) {
-            double ab = 0.0, pb = 0.0;
-            for (int i = 0; i < nk; ++i) {
-                const double s = S[(size_t)i * sstride + e];
-                ab += s * (double)sA[i];
-                pb += s * (double)sP[i];
-            }
-            finish(e, ab, pb);
-        }
-        return wave_sum(rb);
-    }
-    if (qs) {
-        const int t1 = qstart[E];
-        for (int t = lane; t < t1; t += FM_WAVE) {
-            const int i = qorder[t];
-            double gA, gP;
-            adj(i, gA, gP);
-            sA[t] = (T)gA;
-            sP[t] = (T)gP;
-            sF[t] = fq[i];
-            rb += 2.0 * q[i] * gP;
-        }
-        wave_sync();
-        for (int e = lane; e < E; e += FM_WAVE) {
-            double ab = 0.0, pb = 0.0;
-            const int lo0 = qstart[e], lo1 = qstart[e + 1], hi0 = e > 0 ? qstart[e - 1] : lo0;
-            for (int t = lo0; t < lo1; ++t) {
-                ab += (1.0 - sF[t]) * (double)sA[t];
-                pb += (1.0 - sF[t]) * (double)sP[t];
-            }
-            for (int t = hi0; t < lo0; ++t) {
-                ab += sF[t] * (double)sA[t];
-                pb += sF[t] * (double)sP[t];
-            }
-            finish(e, ab, pb);
-        }
-        return wave_sum(rb);
-    }
-    for (int e = lane; e < E; e += FM_WAVE) {
-        double ab = 0.0, pb = 0.0;
-        for (int t = qstart[e]; t < qstart[e + 1]; ++t) {    // q points with lower interpolation energy e
-            const int i = qorder[t];
-            double gA, gP;
-            adj(i, gA, gP);
-            ab += (1.0 - fq[i]) * gA;
-            pb += (1.0 - fq[i]) * gP;
-            rb += 2.0 * q[i] * gP;
-        }
-        if (e > 0)
-            for (int t = qstart[e - 1]; t < qstart[e]; ++t) {  // ... and upper interpolation energy e
-                const int i = qorder[t];
-                double gA, gP;
-                adj(i, gA, gP);
-                ab += fq[i] * gA;
-                pb += fq[i] * gP;
-            }
-        finish(e, ab, pb);
-    }
-    return wave_sum(rb);
 }
 
 template <class T, int SET, int WPE>
@@ -1363,15 +791,10 @@ __device__ __forceinline__ cx<T> ss_fused_energy(const fm_edge &ed, const PathLD
     return pt.v * cfac_at<T>(ed, g, ee, 2);
 }
 
-// The fused adjoint of multiple-scattering paths of NL legs: per band of energies one sweep (fused_energy) that
-// leaves cchi in LDS and the complex derivatives of ptrac in the band's workspace; then per path the fine-grid
-// adjoint (or the given dL/dcchi), pbc and the cfac terms per energy; then the derivative slots contracted with pbc
-// and summed over the energies in band order, and the geometry adjoint.
-// The fused adjoint's sweep (one wavefront per SIMD): per block of G paths, the geometry and the rotation tables
-// with their beta derivatives into LDS, then every energy of every path in one sweep. Each path leaves cchi and the
-// 4 nleg complex derivative slots of every energy in its workspace region (path-major: cchi [E], slot s at
-// [(1 + s) E]); k_adjoint_tail takes it from there. Lanes past their band's end and paths past the launch's end
-// compute on a duplicate and write their slots to the spare region after the last path.
+// The single-scattering adjoint's sweep: per block of G paths the geometry into LDS, then every energy of every path.
+// Each path leaves cchi and the 4 nleg complex derivative slots of every energy in its workspace region (path-major:
+// cchi [E], slot s at [(1 + s) E]); k_adjoint_tail takes it from there. Lanes past their band's end and paths past the
+// launch's end compute on a duplicate and write their slots to the spare region after the last path.
 template <class T, int SET, int NL, int WPE>
 __global__ __launch_bounds__(FM_WAVE * 4) __attribute__((amdgpu_waves_per_eu(WPE))) void k_adjoint(BArgs a) {
     extern __shared__ __align__(16) unsigned char smem[];
@@ -1380,13 +803,10 @@ __global__ __launch_bounds__(FM_WAVE * 4) __attribute__((amdgpu_waves_per_eu(WPE
     const int lane = lane_id();
     const fm_edge &ed = a.ed;
     const int G = a.gp, cap = FM_WAVE / G;
-    const int ltab = ed.L1 + 1, E = ed.E;
+    const int E = ed.E;
     const int nband = a.bp.nband;
     const int jl = lane / cap, il = lane % cap;
-    unsigned char *pbase = smem + (size_t)jl * a.path_bytes;
-    const PathLDS &gj = *reinterpret_cast<const PathLDS *>(pbase);
-    const T *Wj = reinterpret_cast<const T *>(pbase + a.off_W);
-    const T *Wdj = reinterpret_cast<const T *>(pbase + a.off_Wd);
+    const PathLDS &gj = *reinterpret_cast<const PathLDS *>(smem + (size_t)jl * a.path_bytes);
     const __amdgpu_buffer_rsrc_t drs = slice_rsrc(a.work, a.dbytes);
     cx<T> *const wcc = reinterpret_cast<cx<T> *>(a.work);
     const int sbytes = E * (int)sizeof(cx<T>);
@@ -1400,42 +820,23 @@ __global__ __launch_bounds__(FM_WAVE * 4) __attribute__((amdgpu_waves_per_eu(WPE
             const int p = a.order ? a.order[a.first + s0] : a.first + s0;
             PathLDS &g = *reinterpret_cast<PathLDS *>(smem + (size_t)(act ? j : 0) * a.path_bytes);
             int ei;
-            load_path_group(a.src, p, g, ei, NL, lane & 15, act, SET < FM_SET_SS);
+            load_path_group(a.src, p, g, ei, NL, lane & 15, act, false);
         }
-        if constexpr (SET < FM_SET_SS) build_tables<T, SET, true, 16>(ed, smem, a.path_bytes, a.off_W, a.off_Wd, wid, 4, G, NL, ltab);
         __syncthreads();
-        // ---- 2. the fused sweep over this wavefront's bands
+        // ---- 2. the sweep over this wavefront's bands
         const int sj = blk * G + jl;
         const bool vj = sj < a.npath_bucket;
-        // this lane's energy in band b, and its path's (a duplicate in the launch for lanes past its end) kept rows
-        auto energy_of = [&](int b) {
-            const int e0 = a.bp.start[b], nb = a.bp.start[b + 1] - e0;
-            return e0 + (il < nb ? il : nb - 1);
-        };
-        auto kept_at = [&](int e) {
-            return reinterpret_cast<const T *>(a.keep) + ((size_t)(vj ? sj : blk * G) * keep_rows<SET>(NL) * E + e) * 2;
-        };
         auto next_band = [&](int b) {
             for (++b; b < nband && a.bp.wave[b] != wid; ++b) {}
             return b;
         };
         for (int b = next_band(-1); b < nband; b = next_band(b)) {
-            const int e = energy_of(b);
-            const bool on = vj && il < a.bp.start[b + 1] - a.bp.start[b];
+            const int e0 = a.bp.start[b], nb = a.bp.start[b + 1] - e0;
+            const int e = e0 + (il < nb ? il : nb - 1);
+            const bool on = vj && il < nb;
             const size_t reg = on ? (size_t)sj : (size_t)a.npath_bucket;
             const DSlots<T> ds{drs, (uint32_t)((reg * a.dstride + E + e) * sizeof(cx<T>)), sbytes, NL};
-            cx<T> c;
-            if constexpr (SET >= FM_SET_SS) {
-                c = ss_fused_energy<T, SET - FM_SET_SS + 1>(ed, gj, e, ds);
-            } else {
-                cx<T> F[NL - 1][FM_NREP];
-                if (a.keep) {
-                    keep_loads<T, SET, NL, 1>(kept_at(e), E, F);
-                } else {
-                    fused_fblocks<T, SET, NL, 1>(ed, gj, Wj, ltab, e, F);
-                }
-                c = fused_energy<T, SET, NL>(ed, gj, Wj, Wdj, ltab, e, ds, F);
-            }
+            const cx<T> c = ss_fused_energy<T, SET - FM_SET_SS + 1>(ed, gj, e, ds);
             if (on) wcc[(size_t)sj * a.dstride + e] = c;
         }
         __syncthreads();
@@ -1651,14 +1052,8 @@ hipError_t launch_fused_nl(BArgs a, long groups, const fm_launch &pol, size_t sh
     return hipGetLastError();
 }
 
-// LDS of one path in k_adjoint: the geometry and the rotation tables with their beta derivatives.
-template <class T, int SET> __host__ void layout_sweep(BArgs &a) {
-    size_t o = align16(sizeof(PathLDS));
-    const size_t tab = SET >= FM_SET_SS ? 0 : align16(sizeof(T) * rot_elems(a.nlegmax, a.ltab));
-    a.off_W = o; o += tab;
-    a.off_Wd = o; o += tab;
-    a.path_bytes = path_stride(o);
-}
+// LDS of one path in k_adjoint: the geometry.
+void layout_sweep(BArgs &a) { a.path_bytes = path_stride(align16(sizeof(PathLDS))); }
 
 // LDS of one wavefront (one path) of k_adjoint_tail.
 template <class T> __host__ void layout_tail(BArgs &a, const fm_edge &ed) {
@@ -1687,21 +1082,19 @@ template <class T, int NL> hipError_t launch_tail(const BArgs &a, hipStream_t st
 
 constexpr size_t FM_DREGION_MAX = (size_t(1) << 31) - 4096;   // the sweep addresses its workspace with 32-bit offsets
 
-// The fused adjoint (multiple scattering of 3..FM_FUSED_MAXLEG legs, single scattering): k_adjoint's sweep, then
-// k_adjoint_tail, over chunks of the bucket of as many paths as the workspace holds regions for (one spare). Single
-// scattering of K edges keeps little in registers: two workgroups per CU (FP32).
+// Single scattering: k_adjoint's sweep, then k_adjoint_tail, over chunks of the bucket of as many paths as the workspace
+// holds regions for (one spare). K edges keep little in registers: two workgroups per CU (FP32).
 template <class T, int SET> hipError_t launch_fused(BArgs &a, const fm_launch &pol, hipStream_t st) {
     const fm_edge &ed = a.ed;
-    const int nl = SET >= FM_SET_SS ? 2 : a.nlegmax;
-    a.dstride = (size_t)(4 * nl + 1) * ed.E;
+    a.dstride = (size_t)9 * ed.E;
     const size_t per = a.dstride * sizeof(cx<T>);
     const size_t room = a.work_bytes < FM_DREGION_MAX ? a.work_bytes : FM_DREGION_MAX;
     const long chunk = (long)(room / per) - 1;
     if (chunk < 1) return hipErrorOutOfMemory;
     BArgs A = a, B = a;
-    layout_sweep<T, SET>(A);
+    layout_sweep(A);
     size_t budget = fm_lds_budget(sizeof(T) == 4 ? 1 : 3);
-    if (SET >= FM_SET_SS && budget > FM_LDS_SHARE) budget = FM_LDS_SHARE;
+    if (budget > FM_LDS_SHARE) budget = FM_LDS_SHARE;
     const int g = choose_gpaths(ed, A.path_bytes, budget, pol.gpaths);
     if (g == -2) return hipErrorInvalidConfiguration;
     if (g < 0) return hipErrorInvalidValue;
@@ -1710,44 +1103,46 @@ template <class T, int SET> hipError_t launch_fused(BArgs &a, const fm_launch &p
     const size_t shm = A.path_bytes * A.gp;
     layout_tail<T>(B, ed);
     if (B.path_bytes * 4 > FM_LDS_MAX) return hipErrorInvalidValue;
-    // bytes per path of the kept matrices
-    const size_t keep_path = SET >= FM_SET_SS ? 0 : (size_t)ed.E * keep_rows<SET>(nl) * 2 * sizeof(T);
     for (long c0 = 0; c0 < a.npath_bucket; c0 += chunk) {
         const int cnt = (int)(a.npath_bucket - c0 < chunk ? a.npath_bucket - c0 : chunk);
-        A.keep = a.keep ? (const unsigned char *)a.keep + (size_t)c0 * keep_path : nullptr;
         A.first = B.first = a.first + (int)c0;
         A.npath_bucket = B.npath_bucket = cnt;
         A.dbytes = B.dbytes = (size_t)(cnt + 1) * per;
         const long groups = (cnt + A.gp - 1) / A.gp;
         hipError_t e;
-        if constexpr (SET >= FM_SET_SS) {
-            // K: two workgroups per CU; L and M (27 and 21 representatives) would spill at that register budget
-            if (sizeof(T) == 4 && SET == FM_SET_SS && shm <= FM_LDS_SHARE - 256) e = launch_fused_nl<T, SET, 2, 2>(A, groups, pol, shm, st);
-            else e = launch_fused_nl<T, SET, 2, 1>(A, groups, pol, shm, st);
-            if (e == hipSuccess) e = launch_tail<T, 2>(B, st);
-        } else {
-            switch (a.nlegmax) {
-                case 3: e = launch_fused_nl<T, SET, 3>(A, groups, pol, shm, st); if (e == hipSuccess) e = launch_tail<T, 3>(B, st); break;
-                case 4: e = launch_fused_nl<T, SET, 4>(A, groups, pol, shm, st); if (e == hipSuccess) e = launch_tail<T, 4>(B, st); break;
-                case 5: e = launch_fused_nl<T, SET, 5>(A, groups, pol, shm, st); if (e == hipSuccess) e = launch_tail<T, 5>(B, st); break;
-                case 6: e = launch_fused_nl<T, SET, 6>(A, groups, pol, shm, st); if (e == hipSuccess) e = launch_tail<T, 6>(B, st); break;
-                default: e = hipErrorInvalidValue;
-            }
-        }
+        // K: two workgroups per CU; L and M (27 and 21 representatives) would spill at that register budget
+        if (sizeof(T) == 4 && SET == FM_SET_SS && shm <= FM_LDS_SHARE - 256) e = launch_fused_nl<T, SET, 2, 2>(A, groups, pol, shm, st);
+        else e = launch_fused_nl<T, SET, 2, 1>(A, groups, pol, shm, st);
+        if (e == hipSuccess) e = launch_tail<T, 2>(B, st);
         if (e != hipSuccess) return e;
     }
     return hipSuccess;
 }
 
-// Multiple scattering of more than FM_FUSED_MAXLEG legs: pass A stores the prefix products in the workspace, pass B
-// reads them (k_backward). Everything else: the fused adjoint.
+// Multiple scattering of up to FM_FUSED_MAXLEG legs: ms_adjoint (fm_adjoint.hip); of more: pass A stores the prefix
+// products in the workspace, pass B reads them (k_backward). Single scattering: the sweep and its tail.
 template <class T, int SET> hipError_t launch_backward(BArgs &a, const fm_launch &pol, hipStream_t st) {
     const fm_edge &ed = a.ed;
     a.ltab = ed.L1 + 1;
     if constexpr (SET >= FM_SET_SS) {
         return launch_fused<T, SET>(a, pol, st);
     } else {
-        if (a.nlegmax >= 3 && a.nlegmax <= FM_FUSED_MAXLEG) return launch_fused<T, SET>(a, pol, st);
+        if (a.nlegmax >= 3 && a.nlegmax <= FM_FUSED_MAXLEG) {
+            MsAdjoint m;
+            memset(&m, 0, sizeof m);
+            m.ed = ed;
+            m.npath = a.npath_bucket; m.first = a.first; m.edge_id = a.edge_id; m.nleg = a.nlegmax;
+            m.order = a.order;
+            m.src = a.src;
+            m.gcchi = a.gcchi; m.greff = a.greff;
+            m.G = a.G;
+            m.segment = a.segment; m.gseg = a.gseg; m.gpath = a.gpath;
+            m.gcoord = a.gcoord;
+            m.nslot = a.nslot; m.nk = a.nk;
+            m.work = a.work; m.work_bytes = a.work_bytes;
+            m.keep = a.keep;
+            return ms_adjoint(sizeof(T) * 8, m, pol, st);
+        }
         layout<T, SET>(a, ed);
         const int g = choose_gpaths(ed, a.path_bytes, fm_lds_budget(sizeof(T) == 4 ? 1 : 3), pol.gpaths);
         if (g == -2) return hipErrorInvalidConfiguration;
@@ -1826,7 +1221,12 @@ size_t fm_backward_workspace_bytes(int32_t precision, int32_t nlegmax, int32_t b
     const size_t nslots = nlegmax > 2 ? nlegmax - 1 : 1;
     const size_t cxe = nslots * 36 + (size_t)(nlegmax - 1) * FM_NREP;
     const size_t per = (ec * cxe * FM_WAVE + er * (size_t)nacc(nlegmax) * FM_WAVE + 255) & ~size_t(255);
-    return per * (size_t)band_slots;
+    size_t bytes = per * (size_t)band_slots;
+    for (int n = 3; n <= FM_FUSED_MAXLEG && n <= nlegmax; ++n) {   // 16 paths of 3-6 legs at the largest E
+        const size_t b16 = ms_adjoint_bytes16(precision, n);
+        if (b16 > bytes) bytes = b16;
+    }
+    return bytes;
 }
 
 int fm_cchi_backward(const fm_edge *edge, int32_t precision, int32_t iorder, int32_t npath, int32_t nleg,

@@ -22,6 +22,7 @@
 #include <type_traits>
 
 #include "fm_device.h"
+#include "fm_internal.h"
 #include "fm_path.h"
 
 using namespace fm;
@@ -172,6 +173,56 @@ __global__ __launch_bounds__(FM_WAVE * 4) __attribute__((amdgpu_waves_per_eu(FM_
     release_groups(a.tickets);
 }
 
+// The scattering matrices alone, in the kept rows' layout (for an adjoint whose forward kept none): k_forward's setup
+// and bands without the termination and the chain.
+template <class T, int SET>
+__global__ __launch_bounds__(FM_WAVE * 4) __attribute__((amdgpu_waves_per_eu(FM_WPE(T)))) void k_matrices(KArgs a) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    constexpr int L = lamdef(SET).L, L0 = lamdef(SET).L0;
+    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / FM_WAVE);
+    const int lane = lane_id();
+    const fm_edge &ed = a.ed;
+    const int G = a.gp, cap = FM_WAVE / G;
+    const int ltab = ed.L1 + 1, E = ed.E, n = a.nleg, blk = blockIdx.x;
+    const size_t off_W = align16(sizeof(PathLDS));
+    const int jl = lane / cap, il = lane % cap;      // this lane's path and energy within a band
+    unsigned char *lbase = smem + (size_t)jl * a.path_bytes;
+    const PathLDS &g = *reinterpret_cast<const PathLDS *>(lbase);
+    const T *W = reinterpret_cast<const T *>(lbase + off_W);
+    for (int j = wid; j < G; j += 4) {
+        const int slot = blk * G + j;
+        const int s0 = slot < a.npath_bucket ? slot : blk * G;
+        int ei;
+        load_path(a.src, a.order ? a.order[a.first + s0] : a.first + s0,
+                  *reinterpret_cast<PathLDS *>(smem + (size_t)j * a.path_bytes), ei, n);
+    }
+    build_tables<T, SET, false, 1>(ed, smem, a.path_bytes, off_W, 0, wid, 4, G, n, ltab);
+    __syncthreads();
+    const int tlstride = 2 * E;
+    const bool valid = blk * G + jl < a.npath_bucket;
+    for (int b = 0; b < a.bp.nband; ++b) {
+        if (a.bp.wave[b] != wid) continue;
+        const int e0 = a.bp.start[b], nb = a.bp.start[b + 1] - e0;
+        const bool active = il < nb && valid;
+        const int e = e0 + (il < nb ? il : nb - 1);
+        T *kp = reinterpret_cast<T *>(a.keep) + ((size_t)(blk * G + (valid ? jl : 0)) * keep_rows<SET>(n) * E + e) * 2;
+        const cx<T> ck = mk<T>((T)ed.ck[2 * e], (T)ed.ck[2 * e + 1]);
+        auto block = [&](int s, auto nr, auto nc) {
+            constexpr int NR = decltype(nr)::value, NC = decltype(nc)::value;
+            const int ip = g.ipot[s];
+            const T *tl = TL<T>::tl(ed) + ((size_t)ip * ltab) * tlstride + 2 * e;
+            cx<T> Ft[FM_NREP];
+            fblock<T, SET, NR, NC, true>(Ft, ck, (T)g.r[s + 1], (T)g.r[s], ed.lmax[(size_t)ip * E + e] + 1,
+                                         W + (size_t)(s - 1) * ltab * FM_NREP, tl, tlstride);
+            if (active) keep_store<T, SET, NR, NC>(kp + (size_t)2 * E * keep_off<SET>(n, s), E, Ft);
+        };
+        block(1, std::integral_constant<int, L>{}, std::integral_constant<int, L0>{});
+#pragma unroll 1
+        for (int s = 2; s < n - 1; ++s) block(s, std::integral_constant<int, L>{}, std::integral_constant<int, L>{});
+        block(n - 1, std::integral_constant<int, L0>{}, std::integral_constant<int, L>{});
+    }
+}
+
 // GPUPathStage.chi_fine on its own: one wave per path reads cchi [npath][E] and runs the fine-grid epilogue.
 template <class T>
 __global__ __launch_bounds__(FM_WAVE *WPB_MAX) void k_chi_fine(fm_edge ed, int npath, const T *cchi, const double *reff,
@@ -227,6 +278,25 @@ template <class T, int SET> hipError_t launch_forward(KArgs &a, const fm_launch 
     return hipGetLastError();
 }
 
+template <class T, int SET> hipError_t launch_matrices(KArgs &a, const fm_launch &pol, hipStream_t st) {
+    const fm_edge &ed = a.ed;
+    a.path_bytes = path_stride(align16(sizeof(PathLDS)) + align16(sizeof(T) * rot_elems(a.nleg, ed.L1 + 1)));
+    const int g = choose_gpaths(ed, a.path_bytes, fm_lds_budget(sizeof(T) == 4 ? 0 : 2), pol.gpaths);
+    if (g == -2) return hipErrorInvalidConfiguration;
+    if (g < 0) return hipErrorInvalidValue;
+    a.gp = 1 << g;
+    a.bp = ed.bands[g];
+    const size_t shm = a.path_bytes * a.gp;
+    if (shm > 64 * 1024) {
+        hipError_t e = hipFuncSetAttribute((const void *)k_matrices<T, SET>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                           (int)shm);
+        if (e != hipSuccess) return e;
+    }
+    hipLaunchKernelGGL((k_matrices<T, SET>), dim3((unsigned)((a.npath_bucket + a.gp - 1) / a.gp)), dim3(FM_WAVE * 4), shm,
+                       st, a);
+    return hipGetLastError();
+}
+
 template <class T> hipError_t dispatch(KArgs &a, int set, const fm_launch &pol, hipStream_t st) {
     switch (set) {
         case 0: return launch_forward<T, 0>(a, pol, st);
@@ -260,6 +330,22 @@ int check_edge(const fm_edge *e) {
 }
 
 }  // namespace
+
+hipError_t fm::forward_matrices(int precision, const fm_edge &ed, const PathSrc &src, const int32_t *order, int first,
+                                int npath, int nleg, void *keep, const fm_launch &pol, hipStream_t st) {
+    KArgs a;
+    memset(&a, 0, sizeof a);
+    a.ed = ed;
+    a.src = src;
+    a.npath_bucket = npath;
+    a.first = first;
+    a.order = order;
+    a.nleg = nleg;
+    a.keep = keep;
+    if (set_for(ed, nleg) == 0)
+        return precision == 32 ? launch_matrices<float, 0>(a, pol, st) : launch_matrices<double, 0>(a, pol, st);
+    return precision == 32 ? launch_matrices<float, 1>(a, pol, st) : launch_matrices<double, 1>(a, pol, st);
+}
 
 extern "C" {
 

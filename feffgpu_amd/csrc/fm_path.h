@@ -520,16 +520,20 @@ template <> struct TL<double> {
 // cfac = exp(i R (ck - xk)) / prod_j (ck r_j), R = sum r_j = 2 reff (src/feffgpu/stage.py:336-337); the phase
 // R Re(ck - xk) in FP64 reduced mod 2 pi
 template <class T>
-__device__ __forceinline__ cx<T> cfac_at(const fm_edge &ed, const PathLDS &g, int ee, int n) {
+__device__ __forceinline__ cx<T> cfac_of(const fm_edge &ed, double R, double prod_r, int ee, int n) {
     const cx<T> ck = mk<T>((T)ed.ck[2 * ee], (T)ed.ck[2 * ee + 1]);
-    double phs = g.R * ed.ckmxk[2 * ee];
+    double phs = R * ed.ckmxk[2 * ee];
     phs -= FM_TWO_PI * rint(phs / FM_TWO_PI);
-    const double damp = exp(-g.R * ed.ckmxk[2 * ee + 1]);
+    const double damp = exp(-R * ed.ckmxk[2 * ee + 1]);
     T sp, cp;
     if constexpr (sizeof(T) == 4) sincosf((float)phs, &sp, &cp); else sincos(phs, &sp, &cp);
     cx<T> ckn = ck;
     for (int j = 1; j < n; ++j) ckn = ckn * ck;
-    return cdiv(mk<T>((T)damp * cp, (T)damp * sp), ckn * (T)g.prod_r);
+    return cdiv(mk<T>((T)damp * cp, (T)damp * sp), ckn * (T)prod_r);
+}
+template <class T>
+__device__ __forceinline__ cx<T> cfac_at(const fm_edge &ed, const PathLDS &g, int ee, int n) {
+    return cfac_of<T>(ed, g.R, g.prod_r, ee, n);
 }
 
 // cchi at energy e of the path held in g (tables in W). All lanes of the wave run it (e may be out of range for
@@ -560,11 +564,11 @@ __host__ __device__ constexpr KeepList keep_list(int set, int nr, int nc) {
 }
 // rows before scatterer s's block for a path of n legs (run-time n and s; the block sizes are compile-time
 // constants), and the rows of a path
-template <int SET> __host__ __device__ inline int keep_off(int n, int s) {
+template <int SET> __host__ __device__ constexpr int keep_off(int n, int s) {
     constexpr int c1 = keep_count(SET, lamdef(SET).L, lamdef(SET).L0), cm = keep_count(SET, lamdef(SET).L, lamdef(SET).L);
     return s == 1 ? 0 : c1 + (s - 2) * cm;
 }
-template <int SET> __host__ __device__ inline int keep_rows(int n) {
+template <int SET> __host__ __device__ constexpr int keep_rows(int n) {
     constexpr int cl = keep_count(SET, lamdef(SET).L0, lamdef(SET).L);
     return keep_off<SET>(n, n - 1) + cl;
 }

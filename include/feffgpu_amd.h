@@ -125,9 +125,11 @@ int fm_cchi_backward_noalloc(const fm_edge *edge, int32_t precision, int32_t ior
 /* Bytes of the workspace the adjoints need for `band_slots` energy bands of paths of at most nlegmax legs in flight
  * at once (paths of 7-9 legs: each lane keeps its scattering matrices, prefix products and gradient terms there; a
  * workgroup holds one slot per band of its plan, at most 16, and a launch uses as many workgroups as the workspace
- * holds). The adjoint of 2-6 legs keeps (4 nleg + 1) E complex per path (cchi and the derivative slots of every
- * energy) for as many paths of a bucket at a time as the workspace holds regions for, less one spare: larger buckets
- * run in chunks. Any workspace of at least fm_backward_workspace_bytes(precision, nlegmax, 16) bytes works. */
+ * holds). The adjoint of 3-6 legs keeps, per path of a launch, cchi and nleg + 3 derivatives of every energy, the
+ * chain's matrix of every scatterer (up to 20 entries per energy), a record of 14 nleg + 165 numbers and, where the
+ * forward kept none, the scattering matrices; single scattering cchi and 8 derivatives of every energy. Both take as
+ * many paths of a bucket at a time as the workspace holds: larger buckets run in chunks. Any workspace of at least
+ * fm_backward_workspace_bytes(precision, nlegmax, 16) bytes works. */
 size_t fm_backward_workspace_bytes(int32_t precision, int32_t nlegmax, int32_t band_slots);
 
 /* GPUPathStage.chi_fine with the linear ("feff") convention (src/feffgpu/stage.py:365-388): chi [npath][nk] =
