@@ -199,7 +199,9 @@ def backward_workspace(precision: int, nlegmax: int, npath: int, device, E: int,
     slots = max(16, min(int(max_slots), 16 * max(int(npath), 1))) if nlegmax > 6 else 16
     nbytes = lib().fm_backward_workspace_bytes(int(precision), int(nlegmax), slots)
     n, ec = min(int(nlegmax), 6), 8 if precision == 32 else 16
-    per = (40 * (n - 1) + 1) * (int(E) + 3) * ec + 8 * (10 * n + 3)
+    per = 9 * int(E) * ec
+    if n > 2:
+        per = max(per, (40 * (n - 1) + n + 4) * (int(E) + 3) * ec + 8 * (10 * n + 5) + ec // 2 * (4 * n + 160))
     nbytes = max(nbytes, min((int(npath) + 32) * per, int(max_region_bytes)))
     return torch.empty(max(nbytes, 1), dtype=torch.uint8, device=device)
 
