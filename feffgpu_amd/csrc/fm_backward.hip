@@ -1095,7 +1095,8 @@ template <class T, int SET> hipError_t launch_fused(BArgs &a, const fm_launch &p
     layout_sweep(A);
     size_t budget = fm_lds_budget(sizeof(T) == 4 ? 1 : 3);
     if (budget > FM_LDS_SHARE) budget = FM_LDS_SHARE;
-    const int g = choose_gpaths(ed, A.path_bytes, budget, pol.gpaths);
+    const int g = choose_gpaths(ed, A.path_bytes, budget, pol.gpaths, a.npath_bucket < chunk ? a.npath_bucket : chunk,
+                                sizeof(T) == 4 && SET == FM_SET_SS ? 2 : 1);
     if (g == -2) return hipErrorInvalidConfiguration;
     if (g < 0) return hipErrorInvalidValue;
     A.gp = 1 << g;

@@ -258,7 +258,8 @@ template <class T, int SET> hipError_t launch_forward(KArgs &a, const fm_launch 
     a.path_bytes = path_stride(align16(sizeof(PathLDS)) +
                                (SET < FM_SET_SS ? align16(sizeof(T) * rot_elems(a.nleg, ed.L1 + 1)) : 0) +
                                align16(sizeof(T) * ed.E) + align16(sizeof(double) * ed.E));
-    const int g = choose_gpaths(ed, a.path_bytes, fm_lds_budget(sizeof(T) == 4 ? 0 : 2), pol.gpaths);
+    const int g = choose_gpaths(ed, a.path_bytes, fm_lds_budget(sizeof(T) == 4 ? 0 : 2), pol.gpaths,
+                                a.npath_bucket, FM_WPE(T));
     if (g == -2) return hipErrorInvalidConfiguration;
     if (g < 0) return hipErrorInvalidValue;
     a.gp = 1 << g;
@@ -281,7 +282,8 @@ template <class T, int SET> hipError_t launch_forward(KArgs &a, const fm_launch 
 template <class T, int SET> hipError_t launch_matrices(KArgs &a, const fm_launch &pol, hipStream_t st) {
     const fm_edge &ed = a.ed;
     a.path_bytes = path_stride(align16(sizeof(PathLDS)) + align16(sizeof(T) * rot_elems(a.nleg, ed.L1 + 1)));
-    const int g = choose_gpaths(ed, a.path_bytes, fm_lds_budget(sizeof(T) == 4 ? 0 : 2), pol.gpaths);
+    const int g = choose_gpaths(ed, a.path_bytes, fm_lds_budget(sizeof(T) == 4 ? 0 : 2), pol.gpaths,
+                                a.npath_bucket, FM_WPE(T));
     if (g == -2) return hipErrorInvalidConfiguration;
     if (g < 0) return hipErrorInvalidValue;
     a.gp = 1 << g;

@@ -92,15 +92,25 @@ inline int pick_gpaths(const fm_edge &e, size_t path_bytes, size_t budget) {
 }
 
 // log2 of the paths per workgroup of a launch: `want` (1, 2, 4 or 8) if it has a band plan and fits one CU's LDS
-// (-2 if not), else (want 0) the largest within `budget`, else the largest that fits one CU (-1 if none).
-inline int choose_gpaths(const fm_edge &e, size_t path_bytes, size_t budget, int want) {
+// (-2 if not), else (want 0) the largest within `budget`, else the largest that fits one CU (-1 if none), less for a
+// launch of few paths (npath; 0: any number). More paths per workgroup waste fewer lanes on the uneven partial waves,
+// which counts once the chip is full; before that the time is one workgroup's, and fewer paths in it mean fewer paths
+// set up and fewer bands run by each wavefront one after the other. The line: as long as every CU still gets about one
+// workgroup (up to 256 of them; 4 paths up to 320 where two share a CU: resident = 2, FP32). Forward, FP32, us, 8 / 4 / 2 paths per workgroup: K edge,
+// 3 legs, 60 paths 66 / 42 / 40, 600 paths 63 / 40 / 42, 1200 paths 61 / 45 / 79, 2400 paths 71 / 84 / 126; L3, 4 legs,
+// 60 paths 89 / 55 / 52, 1200 paths 87 / 70 / 114; single scattering, 60 paths 30 / 22 / 20, 2400 paths 32 / 36 / 50;
+// FP64, K edge, 3 legs, 60 paths 69 / 43 / 40, 600 paths 65 / 41 / 71, 1200 paths 63 / 73 / 106.
+inline int choose_gpaths(const fm_edge &e, size_t path_bytes, size_t budget, int want, long npath = 0, int resident = 1) {
     if (want > 0) {
         const int g = want == 1 ? 0 : want == 2 ? 1 : want == 4 ? 2 : want == 8 ? 3 : -1;
         if (g < 0 || e.bands[g].nband == 0 || (path_bytes << g) > FM_LDS_MAX - 256) return -2;
         return g;
     }
-    const int g = pick_gpaths(e, path_bytes, budget - 256);
-    return g >= 0 ? g : pick_gpaths(e, path_bytes, FM_LDS_MAX - 256);
+    int g = pick_gpaths(e, path_bytes, budget - 256);
+    if (g < 0) g = pick_gpaths(e, path_bytes, FM_LDS_MAX - 256);
+    if (npath > 0 && g > 2 && e.bands[2].nband > 0 && (npath + 3) / 4 <= (resident > 1 ? 320 : 256)) g = 2;
+    if (npath > 0 && g > 1 && e.bands[1].nband > 0 && (npath + 1) / 2 <= 256) g = 1;
+    return g;
 }
 
 // Workgroups of a launch over `groups` path groups: one per group (grid 0), or a persistent grid of `grid`
