@@ -240,8 +240,97 @@ __global__ __launch_bounds__(FM_WAVE *WPB_MAX) void k_chi_fine(fm_edge ed, int n
             ang[e] = (double)atan2(ci, cr);
         }
         wave_sync();
-        fine_grid<T>(ed, G.jq, G.fq, G.q, G.nk, reff[p], 0.0, amp, ang, chi + (size_t)p * G.nk, G.S, G.sstride);
+        fine_grid<T>(ed, G.jq, G.fq, G.q, G.nk, reff[p], 0.0, amp, ang, chi + (size_t)p * G.nk);
         wave_sync();
+    }
+}
+
+// The same with a dense interpolation matrix S [nk][sstride]: a contraction of S with the amplitudes and phases of 64
+// paths per workgroup, lanes over the paths, DR rows of S per wavefront. S is wave-uniform (scalar loads, an operand of
+// the FP64 multiply-adds), the amplitudes and phases come from LDS, DE energies at a time, and are read once per DR
+// rows; the sums run over the energies in order, as in fine_grid. Bound by the latency of the scalar loads and of the
+// amplitudes (few wavefronts: DR = 4). One wavefront per path with the lanes over the rows (k_chi_fine) reads all of S
+// per path, a cache line per lane and energy: 2048 paths, E = 59, nk = 361, FP32: 96 us, here 19 us (DR = 8: 25).
+constexpr int DR = 4, DW = 8, DE = 64, DLD = FM_WAVE + 1;
+typedef const __attribute__((address_space(4))) double *scalar_ptr;
+template <class T>
+__global__ __launch_bounds__(FM_WAVE *DW) void k_chi_dense(fm_edge ed, int npath, const T *cchi, const double *reff,
+                                                           fm_grid G, T *chi) {
+    __shared__ T amp[DE * DLD];
+    __shared__ double ang[DE * DLD], tot[DW][FM_WAVE];
+    static_assert(DE == 8 * DW, "8 energies per wavefront");
+    const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / FM_WAVE), lane = lane_id();
+    const int E = ed.E, p0 = blockIdx.x * FM_WAVE, np = npath - p0 < FM_WAVE ? npath - p0 : FM_WAVE;
+    const int i0 = (blockIdx.y * DW + wid) * DR;
+    double sa[DR], sp[DR];
+    scalar_ptr Sr[DR];
+#pragma unroll
+    for (int r = 0; r < DR; ++r) {
+        sa[r] = sp[r] = 0.0;
+        const int i = i0 + r < G.nk ? i0 + r : G.nk - 1;
+        Sr[r] = (scalar_ptr)(uintptr_t)(G.S + (size_t)i * G.sstride);
+    }
+    const int j = lane < np ? lane : np - 1;
+    const T *const c0 = cchi + (size_t)(p0 + j) * E * 2;
+    double carry = 0.0;
+    for (int e0 = 0; e0 < E; e0 += DE) {
+        const int ne = E - e0 < DE ? E - e0 : DE;
+        // energies e0 + 8 wid .. + 7 of path `lane`: amplitudes, and the phase steps wrapped to (-pi, pi], summed over
+        // the thread's 8 and then over the wavefronts
+        double d[8], last = 0.0;
+        {
+            const int eb = e0 + wid * 8;
+            const T *cp = c0 + 2 * (size_t)(eb > 0 ? (eb <= E ? eb - 1 : E - 1) : 0);
+            last = eb > 0 ? (double)atan2(cp[1], cp[0]) : 0.0;
+            double s = 0.0;
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                const int e = eb + u < E ? eb + u : E - 1;
+                const T cr = c0[2 * (size_t)e], ci = c0[2 * (size_t)e + 1];
+                amp[(wid * 8 + u) * DLD + lane] = (T)sqrt((double)cr * cr + (double)ci * ci + 1e-30);
+                const double a = (double)atan2(ci, cr), x = a - last;
+                s += eb + u == 0 ? a : eb + u < E ? x - FM_TWO_PI * rint(x / FM_TWO_PI) : 0.0;
+                d[u] = s;
+                last = a;
+            }
+            tot[wid][lane] = s;
+        }
+        __syncthreads();
+        double before = carry;
+#pragma unroll
+        for (int w = 0; w < DW; ++w) {
+            if (w < wid) before += tot[w][lane];
+            carry += tot[w][lane];
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u) ang[(wid * 8 + u) * DLD + lane] = before + d[u];
+        __syncthreads();
+        if (i0 < G.nk) {
+#pragma unroll 4
+            for (int e = 0; e < ne; ++e) {
+                const double av = (double)amp[e * DLD + lane], pv = ang[e * DLD + lane];
+#pragma unroll
+                for (int r = 0; r < DR; ++r) {
+                    const double s = Sr[r][e0 + e];
+                    sa[r] += s * av;
+                    sp[r] += s * pv;
+                }
+            }
+        }
+        __syncthreads();
+    }
+    if (lane >= np) return;
+    const double R = reff[p0 + lane];
+#pragma unroll
+    for (int r = 0; r < DR; ++r) {
+        const int i = i0 + r;
+        if (i >= G.nk) break;
+        double ph = sp[r] + 2.0 * G.q[i] * R;
+        ph -= FM_TWO_PI * rint(ph / FM_TWO_PI);
+        T v;
+        if constexpr (sizeof(T) == 4) v = (T)sa[r] * sinf((float)ph);
+        else v = (T)sa[r] * sin(ph);
+        chi[(size_t)(p0 + lane) * G.nk + i] = v;
     }
 }
 
@@ -411,7 +500,16 @@ int fm_chi_fine(const fm_edge *edge, int32_t precision, int32_t npath, const voi
     const int wpb = WPB_MAX;
     const int blocks = (npath + wpb - 1) / wpb;
     hipStream_t st = (hipStream_t)stream;
-    if (precision == 32)
+    if (grid->S) {
+        const dim3 g((unsigned)((npath + FM_WAVE - 1) / FM_WAVE), (unsigned)((grid->nk + DR * DW - 1) / (DR * DW)));
+        if (grid->nk < 1) return FM_OK;
+        if (precision == 32)
+            hipLaunchKernelGGL(k_chi_dense<float>, g, dim3(FM_WAVE * DW), 0, st, *edge, npath, (const float *)cchi, reff,
+                               *grid, (float *)chi);
+        else
+            hipLaunchKernelGGL(k_chi_dense<double>, g, dim3(FM_WAVE * DW), 0, st, *edge, npath, (const double *)cchi,
+                               reff, *grid, (double *)chi);
+    } else if (precision == 32)
         hipLaunchKernelGGL(k_chi_fine<float>, dim3(blocks), dim3(FM_WAVE * wpb), wb * wpb, st, *edge, npath,
                            (const float *)cchi, reff, *grid, (float *)chi, wb);
     else
