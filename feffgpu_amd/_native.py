@@ -139,6 +139,9 @@ def lib():
         L.fm_find_group_workspace_bytes.argtypes = [_i64]
         L.fm_find_degenerate_total.argtypes = [_i64, _i32, _vp, _vp, _vp, _vp, _vp, _sz, _vp]
         L.fm_find_filter.argtypes = [_i64, _vp, _vp, _vp, _vp, _f32, _vp, _vp]
+        L.fm_find_ref.argtypes = [_i32, _i64, _vp, _vp, _vp, _vp, _vp, _i32, _vp, _vp]
+        L.fm_find_select.argtypes = [_i64, _vp, _vp, _vp, _vp, _f32, _vp, _vp, _vp, _sz, _vp]
+        L.fm_find_compact.argtypes = [_i64, _i32, _vp, _vp, _P(FmFindOut), _vp, _P(FmFindOut), _vp, _vp]
         L.fm_backward_workspace_bytes.restype = ctypes.c_size_t
         L.fm_backward_workspace_bytes.argtypes = [_i32, _i32, _i32]
         L.fm_chi_fine.argtypes = [ctypes.POINTER(FmEdge), _i32, _i32, _vp, _vp, ctypes.POINTER(FmGrid), _vp, _vp]

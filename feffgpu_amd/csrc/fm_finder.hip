@@ -298,14 +298,14 @@ __global__ void k_find_emit(int64_t npart, int32_t m, Partial in, const int32_t 
 }
 
 // Block scan of FD_SCAN_ITEMS counts per block (exclusive, int64), block totals in sums.
-__global__ __launch_bounds__(1024) void k_scan_local(const int32_t *in, int64_t n, int64_t *out, int64_t *sums) {
+template <class In> __global__ __launch_bounds__(1024) void k_scan_local(In in, int64_t n, int64_t *out, int64_t *sums) {
     __shared__ int64_t ws[16];
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const int64_t base = (int64_t)blockIdx.x * FD_SCAN_ITEMS + (int64_t)tid * 4;
     int64_t v[4], s = 0;
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-        v[k] = base + k < n ? in[base + k] : 0;
+        v[k] = base + k < n ? in(base + k) : 0;
         s += v[k];
     }
     int64_t x = s;     // inclusive wave scan of the thread sums
@@ -478,13 +478,75 @@ __global__ void k_find_group_read(int64_t npath, const int64_t *where, const flo
     if (p < npath) total[p] = sums[where[p]];
 }
 
-// keep[p] = 100 dtot xp / ref[slot] >= critpw, in float32 as the reference evaluates it
-__global__ void k_find_filter(int64_t npath, const float *dtot, const float *xp, const int32_t *slot, const float *ref,
-                              float critpw, uint8_t *keep) {
+// 100 dtot xp / ref[slot] >= critpw, in float32 as the reference evaluates it
+struct Filter {
+    const float *dtot, *xp;
+    const int32_t *slot;
+    const float *ref;
+    float critpw;
+    __device__ __forceinline__ int operator()(int64_t p) const {
+        const float frac = ((100.f * dtot[p]) * xp[p]) / ref[slot[p]];
+        return frac >= critpw ? 1 : 0;
+    }
+};
+struct Counts {
+    const int32_t *n;
+    __device__ __forceinline__ int operator()(int64_t p) const { return n[p]; }
+};
+
+__global__ void k_find_filter(int64_t npath, Filter f, uint8_t *keep) {
     const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (p < npath) keep[p] = (uint8_t)f(p);
+}
+
+// The kept paths moved up: row p goes to pos[p] where the next row's pos (past the last row: total) is higher. A thread
+// per (path, atom).
+__global__ void k_find_compact(int64_t npath, int32_t nleg, const int64_t *pos, const int64_t *total, PathOut in,
+                               const float *xin, PathOut out, float *xout) {
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, p = t / nleg;
     if (p >= npath) return;
-    const float frac = ((100.f * dtot[p]) * xp[p]) / ref[slot[p]];
-    keep[p] = frac >= critpw ? 1 : 0;
+    const int j = (int)(t - p * nleg);
+    const int64_t q = pos[p];
+    if ((p + 1 < npath ? pos[p + 1] : *total) == q) return;
+    const size_t a = (size_t)p * nleg + j, b = (size_t)q * nleg + j;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) out.coords[3 * b + c] = in.coords[3 * a + c];
+    out.ipots[b] = in.ipots[a];
+    if (j < nleg - 1) out.atoms[(size_t)q * (nleg - 1) + j] = in.atoms[(size_t)p * (nleg - 1) + j];
+    else {
+        out.deg[q] = in.deg[p];
+        out.slot[q] = in.slot[p];
+        xout[q] = xin[p];
+    }
+}
+
+// ref[b]: the importance of absorber b's shortest two-leg path (the first of equal lengths), times its degeneracy if
+// merged and b has more than one candidate; 1 without paths. The paths are ordered by slot. A wavefront per absorber.
+__global__ void k_find_ref(int32_t nabs, int64_t npath, const int32_t *slot, const float *len, const float *xp,
+                           const float *deg, const int32_t *ncand, int32_t merged, float *ref) {
+    const int b = blockIdx.x, lane = threadIdx.x;
+    auto first = [&](int v) {     // the first path of a slot >= v
+        int64_t lo = 0, hi = npath;
+        while (lo < hi) {
+            const int64_t mid = (lo + hi) / 2;
+            if (slot[mid] < v) lo = mid + 1; else hi = mid;
+        }
+        return lo;
+    };
+    const int64_t s0 = first(b), s1 = first(b + 1);
+    float d = INFINITY;
+    int64_t k = INT64_MAX;
+    for (int64_t p = s0 + lane; p < s1; p += 64) {
+        const float x = len[p];
+        if (k == INT64_MAX || x < d) { d = x; k = p; }
+    }
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) {
+        const float x = __shfl_xor(d, off, 64);
+        const int64_t q = __shfl_xor(k, off, 64);
+        if (q != INT64_MAX && (k == INT64_MAX || x < d || (x == d && q < k))) { d = x; k = q; }
+    }
+    if (lane == 0) ref[b] = s1 > s0 ? (merged && ncand[b] > 1 ? xp[k] * deg[k] : xp[k]) : 1.f;
 }
 
 int launch_err(const char *what) {
@@ -496,6 +558,20 @@ int launch_err(const char *what) {
 }
 
 unsigned blocks_of(int64_t n, int t) { return (unsigned)((n + t - 1) / t); }
+
+template <class In> void run_scan(In in, int64_t n, int64_t *out, int64_t *total, int64_t *sums, hipStream_t st) {
+    const int64_t nb = (n + FD_SCAN_ITEMS - 1) / FD_SCAN_ITEMS;
+    if (nb > 0) hipLaunchKernelGGL(k_scan_local<In>, dim3((unsigned)nb), dim3(1024), 0, st, in, n, out, sums);
+    hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(1024), 0, st, sums, nb, total);
+    if (n > 0) hipLaunchKernelGGL(k_scan_add, dim3(blocks_of(n, 256)), dim3(256), 0, st, out, n, sums);
+}
+
+PathOut path_out(const fm_find_out *o) {
+    PathOut p;
+    memset(&p, 0, sizeof p);
+    if (o) { p.atoms = o->atoms; p.coords = o->coords; p.ipots = o->ipots; p.deg = o->deg; p.slot = o->slot; }
+    return p;
+}
 
 }  // namespace
 
@@ -528,14 +604,10 @@ size_t fm_scan_workspace_bytes(int64_t n) { return sizeof(int64_t) * ((n + FD_SC
 int fm_exclusive_scan(const int32_t *in, int64_t n, int64_t *out, int64_t *total, void *workspace, size_t bytes,
                       void *stream) {
     if (n < 0) return fm_set_err(FM_EINVAL, "fm_exclusive_scan: n < 0");
-    const int64_t nb = (n + FD_SCAN_ITEMS - 1) / FD_SCAN_ITEMS;
-    if (nb > FD_SCAN_ITEMS) return fm_set_err(FM_EINVAL, "fm_exclusive_scan: more than 2^24 items");
+    if ((n + FD_SCAN_ITEMS - 1) / FD_SCAN_ITEMS > FD_SCAN_ITEMS)
+        return fm_set_err(FM_EINVAL, "fm_exclusive_scan: more than 2^24 items");
     if (bytes < fm_scan_workspace_bytes(n)) return fm_set_err(FM_EINVAL, "fm_exclusive_scan: workspace too small");
-    int64_t *sums = (int64_t *)workspace;
-    hipStream_t st = (hipStream_t)stream;
-    if (nb > 0) hipLaunchKernelGGL(k_scan_local, dim3((unsigned)nb), dim3(1024), 0, st, in, n, out, sums);
-    hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(1024), 0, st, sums, nb, total);
-    if (n > 0) hipLaunchKernelGGL(k_scan_add, dim3(blocks_of(n, 256)), dim3(256), 0, st, out, n, sums);
+    run_scan(Counts{in}, n, out, total, (int64_t *)workspace, (hipStream_t)stream);
     return launch_err("fm_exclusive_scan");
 }
 
@@ -546,16 +618,10 @@ int fm_find_write(int32_t nabs, const int32_t *absorbers, const int64_t *off3, c
     if (nabs <= 0 || ncmax <= 0) return FM_OK;
     if (!o2 || (nlegmax >= 3 && (!o3 || !pos3)) || (nlegmax >= 4 && (!o4 || !pos4)))
         return fm_set_err(FM_EINVAL, "fm_find_write: NULL output");
-    auto cv = [](const fm_find_out *o) {
-        PathOut p;
-        memset(&p, 0, sizeof p);
-        if (o) { p.atoms = o->atoms; p.coords = o->coords; p.ipots = o->ipots; p.deg = o->deg; p.slot = o->slot; }
-        return p;
-    };
     const int64_t items = (int64_t)ncmax * (nlegmax >= 4 ? ncmax + 1 : 1);
     hipLaunchKernelGGL(k_find_write, dim3(blocks_of(items, FD_THREADS), nabs), dim3(FD_THREADS), 0, (hipStream_t)stream,
-                       nabs, absorbers, off3, off4, maxc, cidx, crel, cd0, ncand, ipot, 2.f * rmax, nlegmax, off2, cv(o2),
-                       pos3, cv(o3), pos4, cv(o4));
+                       nabs, absorbers, off3, off4, maxc, cidx, crel, cd0, ncand, ipot, 2.f * rmax, nlegmax, off2, path_out(o2),
+                       pos3, path_out(o3), pos4, path_out(o4));
     return launch_err("fm_find_write");
 }
 
@@ -636,9 +702,42 @@ int fm_find_filter(int64_t npath, const float *dtot, const float *xport, const i
                    float critpw, uint8_t *keep, void *stream) {
     if (npath <= 0) return FM_OK;
     if (!dtot || !xport || !slot || !ref || !keep) return fm_set_err(FM_EINVAL, "fm_find_filter: NULL buffer");
-    hipLaunchKernelGGL(k_find_filter, dim3(blocks_of(npath, 256)), dim3(256), 0, (hipStream_t)stream, npath, dtot,
-                       xport, slot, ref, critpw, keep);
+    hipLaunchKernelGGL(k_find_filter, dim3(blocks_of(npath, 256)), dim3(256), 0, (hipStream_t)stream, npath,
+                       Filter{dtot, xport, slot, ref, critpw}, keep);
     return launch_err("fm_find_filter");
+}
+
+int fm_find_ref(int32_t nabs, int64_t npath, const int32_t *slot, const float *len, const float *xport, const float *deg,
+                const int32_t *ncand, int32_t merged, float *ref, void *stream) {
+    if (nabs <= 0) return FM_OK;
+    if (!ref || npath < 0 || (npath > 0 && (!slot || !len || !xport)) || (merged && (!deg || !ncand)))
+        return fm_set_err(FM_EINVAL, "fm_find_ref: bad arguments");
+    hipLaunchKernelGGL(k_find_ref, dim3(nabs), dim3(64), 0, (hipStream_t)stream, nabs, npath, slot, len, xport, deg, ncand,
+                       merged, ref);
+    return launch_err("fm_find_ref");
+}
+
+int fm_find_select(int64_t npath, const float *dtot, const float *xport, const int32_t *slot, const float *ref,
+                   float critpw, int64_t *pos, int64_t *total, void *workspace, size_t bytes, void *stream) {
+    if (npath < 0 || !total || (npath > 0 && (!dtot || !xport || !slot || !ref || !pos)))
+        return fm_set_err(FM_EINVAL, "fm_find_select: bad arguments");
+    if ((npath + FD_SCAN_ITEMS - 1) / FD_SCAN_ITEMS > FD_SCAN_ITEMS)
+        return fm_set_err(FM_EINVAL, "fm_find_select: more than 2^24 paths");
+    if (!workspace || bytes < fm_scan_workspace_bytes(npath))
+        return fm_set_err(FM_EINVAL, "fm_find_select: workspace too small");
+    run_scan(Filter{dtot, xport, slot, ref, critpw}, npath, pos, total, (int64_t *)workspace, (hipStream_t)stream);
+    return launch_err("fm_find_select");
+}
+
+int fm_find_compact(int64_t npath, int32_t nleg, const int64_t *pos, const int64_t *total, const fm_find_out *in,
+                    const float *xport, const fm_find_out *out, float *xport_out, void *stream) {
+    if (npath <= 0) return FM_OK;
+    if (nleg < 2 || nleg > FM_MAX_LEGS || npath > ((int64_t)1 << 24) || !pos || !total || !in || !out || !xport ||
+        !xport_out)
+        return fm_set_err(FM_EINVAL, "fm_find_compact: bad arguments");
+    hipLaunchKernelGGL(k_find_compact, dim3(blocks_of(npath * nleg, 256)), dim3(256), 0, (hipStream_t)stream, npath, nleg,
+                       pos, total, path_out(in), xport, path_out(out), xport_out);
+    return launch_err("fm_find_compact");
 }
 
 }  // extern "C"

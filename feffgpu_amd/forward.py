@@ -226,7 +226,7 @@ class MultipleScattering:
         self.lists = {nleg: dict(atoms=v["atoms"].long(), absorber=ab[v["slot"].long()], ipots=v["ipots"],
                                  deg=v["deg"]) for nleg, v in sorted(kept.items()) if nleg >= 3 and v["deg"].numel()}
         self.C, self.n, self.A, self.n_abs = C, n, A, C * A
-        self.abs_atoms = (absorbers[None, :] + n * torch.arange(C, device=self.device)[:, None]).reshape(-1)
+        self.abs_atoms = ab
         self.row_of = torch.full((C * n,), -1, device=self.device, dtype=torch.long)
         self.row_of[self.abs_atoms] = torch.arange(C * A, device=self.device)
         self.counts = {nleg: int(v["atoms"].shape[0]) for nleg, v in self.lists.items()}

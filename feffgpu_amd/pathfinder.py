@@ -33,6 +33,9 @@ NLEG_MAX = 9
 # absorbers enumerated together: the four-leg counts take nc (nc + 1) int32 per absorber (nc candidates within rmax)
 ABSORBERS_PER_PASS = 4096
 PARTIAL_LIMIT = 30_000_000     # partial paths held per absorber (on average over a call) while 5+-leg paths grow
+SELECT_MAX = 1 << 24           # paths of one pass of the filter's row numbers
+_ROWS = ("atoms", "coords", "ipots", "deg", "slot")
+_KEPT = ("coords", "ipots", "deg", "xport", "atoms", "slot")
 _SEQ = N.FM_MAX_LEGS - 1
 
 
@@ -143,14 +146,28 @@ class GPUPathFinder:
 
     # -- enumeration ------------------------------------------------------------------------------------------
     def _scan(self, cnt):
+        pos, tot = self._scan_all([cnt])
+        return pos[0], tot[0]
+
+    def _scan_all(self, cnts):
+        """The exclusive scan of every int32 vector in ``cnts`` and their sums: one read-back for all."""
         L = N.lib()
-        n = cnt.numel()
-        pos = torch.empty(n, dtype=torch.int64, device=self.device)
-        total = torch.zeros(1, dtype=torch.int64, device=self.device)
-        ws = torch.empty(int(L.fm_scan_workspace_bytes(n)), dtype=torch.uint8, device=self.device)
-        N.check(L.fm_exclusive_scan(cnt.data_ptr(), n, pos.data_ptr(), total.data_ptr(), ws.data_ptr(), ws.numel(),
-                                    N.stream_of(self.device)), "fm_exclusive_scan")
-        return pos, int(total.item())
+        total = torch.empty(len(cnts), dtype=torch.int64, device=self.device)
+        out = []
+        for i, cnt in enumerate(cnts):
+            n = cnt.numel()
+            pos = torch.empty(n, dtype=torch.int64, device=self.device)
+            ws = torch.empty(int(L.fm_scan_workspace_bytes(n)), dtype=torch.uint8, device=self.device)
+            N.check(L.fm_exclusive_scan(cnt.data_ptr(), n, pos.data_ptr(), total.data_ptr() + 8 * i, ws.data_ptr(),
+                                        ws.numel(), N.stream_of(self.device)), "fm_exclusive_scan")
+            out.append(pos)
+        return out, total.tolist()
+
+    @staticmethod
+    def _out_struct(t):
+        s = N.FmFindOut()
+        s.atoms, s.coords, s.ipots, s.deg, s.slot = (t[k].data_ptr() for k in _ROWS)
+        return s
 
     def _alloc(self, P, nleg):
         dev = self.device
@@ -159,9 +176,7 @@ class GPUPathFinder:
                  ipots=torch.empty(P, nleg, dtype=torch.int64, device=dev),
                  deg=torch.empty(P, dtype=torch.float32, device=dev),
                  slot=torch.empty(P, dtype=torch.int32, device=dev))
-        s = N.FmFindOut()
-        s.atoms, s.coords, s.ipots, s.deg, s.slot = (t[k].data_ptr() for k in ("atoms", "coords", "ipots", "deg", "slot"))
-        return t, s
+        return t, self._out_struct(t)
 
     def _partials(self, P):
         dev = self.device
@@ -211,8 +226,10 @@ class GPUPathFinder:
         ip = torch.as_tensor(ipot, device=dev).to(torch.int32).reshape(-1).contiguous()
         if ip.numel() != n:
             raise ValueError("ipot needs one potential per atom")
-        if A and (int(ab.min()) < 0 or int(ab.max()) >= n * nconf):
+        if n * nconf == 0:
             raise ValueError("absorber index outside the configurations")
+        # the kernels get the indices clamped; whether that changed any is read back with the candidates' counts
+        given, ab = ab, ab.clamp(0, n * nconf - 1)
         if nconf > 1:
             ip = ip.repeat(nconf)
         sysd = N.FmFindSys()
@@ -227,11 +244,15 @@ class GPUPathFinder:
             cidx = torch.empty(A, maxc, dtype=torch.int32, device=dev)
             crel = torch.empty(A, maxc, 3, dtype=torch.float32, device=dev)
             cd0 = torch.empty(A, maxc, dtype=torch.float32, device=dev)
-            ncand = torch.zeros(max(A, 1), dtype=torch.int32, device=dev)
+            ncand = torch.zeros(A + 1, dtype=torch.int32, device=dev)
+            ncand[A:].copy_((ab != given).any())
             N.check(L.fm_find_candidates(ctypes.byref(sysd), A, ab.data_ptr(), maxc, cidx.data_ptr(), crel.data_ptr(),
                                          cd0.data_ptr(), ncand.data_ptr(), st), "fm_find_candidates")
-            nc = ncand[:A].cpu().numpy().astype(np.int64)
-            if A == 0 or nc.max() <= maxc:
+            nc = ncand.cpu().numpy().astype(np.int64)
+            if nc[A]:
+                raise ValueError("absorber index outside the configurations")
+            nc = nc[:A]
+            if nc.max() <= maxc:
                 break
             maxc = int(nc.max())
         rmax32 = float(np.float32(self.rmax))
@@ -244,12 +265,12 @@ class GPUPathFinder:
         n4 = np.where(multi, nc * (nc + 1), 0)
         off3 = np.concatenate([[0], np.cumsum(n3)])
         off4 = np.concatenate([[0], np.cumsum(n4)])
-        t64 = lambda a: torch.tensor(np.ascontiguousarray(a, np.int64), device=dev)
-        off2_t, off3_t, off4_t = t64(off2), t64(off3), t64(off4)
-        ncmax = int(nc.max()) if A else 0
+        off2_t, off3_t, off4_t = torch.tensor(np.stack([off2, off3, off4]).astype(np.int64), device=dev)
+        ncmax = int(nc.max())
         nlm = self.nlegmax
-        cnt3 = torch.zeros(max(int(off3[-1]), 1), dtype=torch.int32, device=dev)
-        cnt4 = torch.zeros(max(int(off4[-1]), 1), dtype=torch.int32, device=dev)
+        tot3, tot4 = int(off3[-1]), int(off4[-1])
+        cnt3, cnt4 = torch.zeros(max(tot3, 1) + max(tot4, 1), dtype=torch.int32, device=dev).split(
+            [max(tot3, 1), max(tot4, 1)])
         if nlm >= 3 and ncmax > 1:
             N.check(L.fm_find_count(A, off3_t.data_ptr(), off4_t.data_ptr(), maxc, crel.data_ptr(), cd0.data_ptr(),
                                     ncand.data_ptr(), ncmax, rmax32, nlm, cnt3.data_ptr(), cnt4.data_ptr(), st),
@@ -257,10 +278,12 @@ class GPUPathFinder:
         res = {}
         o2, s2 = self._alloc(int(off2[-1]), 2)
         if nlm >= 3:
-            pos3, tot3 = self._scan(cnt3[:max(int(off3[-1]), 0)].contiguous()) if off3[-1] else (cnt3.long(), 0)
+            pos3 = pos4 = cnt3.long()
+            if tot3:      # and then tot4, whose items are those of the same absorbers
+                pos, tot = self._scan_all([cnt3, cnt4][:nlm - 2])
+                pos3, pos4, tot3, tot4 = pos[0], pos[-1], tot[0], tot[-1]
             o3, s3 = self._alloc(tot3, 3)
         if nlm >= 4:
-            pos4, tot4 = self._scan(cnt4[:max(int(off4[-1]), 0)].contiguous()) if off4[-1] else (cnt4.long(), 0)
             o4, s4 = self._alloc(tot4, 4)
         if ncmax > 0:
             N.check(L.fm_find_write(A, ab.data_ptr(), off3_t.data_ptr(), off4_t.data_ptr(), maxc, cidx.data_ptr(),
@@ -322,31 +345,53 @@ class GPUPathFinder:
         ref = np.ones(A, np.float32)
         if self.merge_degenerate and multi.any():
             res[2] = self._merge_single_scattering(res, A, multi)
-        xp2 = res[2]["xport"].cpu().numpy()
-        slot2 = res[2]["slot"].cpu().numpy()
-        d2 = torch.linalg.vector_norm(res[2]["coords"][:, 1], dim=-1).cpu().numpy() if len(slot2) else np.zeros(0)
-        deg2 = res[2]["deg"].cpu().numpy()
-        start = np.searchsorted(slot2, np.arange(A + 1))
-        for b in range(A):
-            s0, s1 = start[b], start[b + 1]
-            if s1 > s0:
-                k = s0 + int(np.argmin(d2[s0:s1]))
-                ref[b] = np.float32(xp2[k] * deg2[k]) if (self.merge_degenerate and multi[b]) else xp2[k]
-        ref_t = torch.tensor(ref, device=dev)
-        kept = {}
+        # the filter in row numbers (SELECT_MAX paths at a time), every list's numbers of kept paths and the reference
+        # importances in one read-back
+        jobs = []
         for nleg, o in res.items():
             P = o["deg"].numel()
-            if nleg > 2 and self.merge_degenerate and P:
-                dtot = self.degenerate_total(o["coords"], o["deg"], o["slot"])
-            else:
-                dtot = o["deg"]
-            keep = torch.empty(P, dtype=torch.uint8, device=dev)
-            if P:
-                N.check(L.fm_find_filter(P, dtot.data_ptr(), o["xport"].data_ptr(), o["slot"].data_ptr(),
-                                         ref_t.data_ptr(), float(np.float32(self.critpw)), keep.data_ptr(), st),
-                        "fm_find_filter")
-            sel = keep.bool()
-            kept[nleg] = {k: o[k][sel] for k in ("coords", "ipots", "deg", "xport", "atoms", "slot")}
+            dtot = (self.degenerate_total(o["coords"], o["deg"], o["slot"])
+                    if nleg > 2 and self.merge_degenerate and P else o["deg"])
+            jobs += [(nleg, dtot, p0, min(P, p0 + SELECT_MAX)) for p0 in range(0, max(P, 1), SELECT_MAX)]
+        back = torch.empty(len(jobs) + (A + 1) // 2, dtype=torch.int64, device=dev)
+        ref_t = back[len(jobs):].view(torch.float32)[:A]
+        o2 = res[2]
+        n2 = o2["deg"].numel()
+        d2 = torch.linalg.vector_norm(o2["coords"][:, 1], dim=-1) if n2 else o2["deg"]
+        N.check(L.fm_find_ref(A, n2, o2["slot"].data_ptr(), d2.data_ptr(), o2["xport"].data_ptr(), o2["deg"].data_ptr(),
+                              ncand.data_ptr(), int(self.merge_degenerate), ref_t.data_ptr(), st), "fm_find_ref")
+        rows = []
+        for i, (nleg, dtot, p0, p1) in enumerate(jobs):
+            o, n = res[nleg], p1 - p0
+            pos = torch.empty(n, dtype=torch.int64, device=dev)
+            ws = torch.empty(int(L.fm_scan_workspace_bytes(n)), dtype=torch.uint8, device=dev)
+            N.check(L.fm_find_select(n, dtot[p0:].data_ptr(), o["xport"][p0:].data_ptr(), o["slot"][p0:].data_ptr(),
+                                     ref_t.data_ptr(), float(np.float32(self.critpw)), pos.data_ptr(),
+                                     back.data_ptr() + 8 * i, ws.data_ptr(), ws.numel(), st), "fm_find_select")
+            rows.append(pos)
+        h = back.cpu().numpy()
+        total, ref = h[:len(jobs)], h[len(jobs):].view(np.float32)[:A].copy()
+        kept = {}
+        for nleg, o in res.items():
+            mine = [i for i, j in enumerate(jobs) if j[0] == nleg]
+            n = int(total[mine].sum())
+            if n == o["deg"].numel():
+                kept[nleg] = {k: o[k] for k in _KEPT}
+                continue
+            t, _ = self._alloc(n, nleg)
+            t["xport"] = torch.empty(n, dtype=torch.float32, device=dev)
+            at = 0
+            for i in mine:
+                if not total[i]:
+                    continue
+                _, _, p0, p1 = jobs[i]
+                a, b = ({k: v[first:] for k, v in w.items()} for first, w in ((p0, o), (at, t)))
+                N.check(L.fm_find_compact(p1 - p0, nleg, rows[i].data_ptr(), back.data_ptr() + 8 * i,
+                                          ctypes.byref(self._out_struct(a)), a["xport"].data_ptr(),
+                                          ctypes.byref(self._out_struct(b)), b["xport"].data_ptr(), st),
+                        "fm_find_compact")
+                at += int(total[i])
+            kept[nleg] = {k: t[k] for k in _KEPT}
         return kept, ref
 
     def _merge_single_scattering(self, res, A, multi):

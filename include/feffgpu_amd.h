@@ -366,6 +366,17 @@ int fm_find_degenerate_total(int64_t npath, int32_t nleg, const float *coords, c
 /* The importance filter (pathfinder.py:272-278): keep[p] = 100 dtot xp / ref[slot] >= critpw, in float32. */
 int fm_find_filter(int64_t npath, const float *dtot, const float *xport, const int32_t *slot, const float *ref,
                    float critpw, uint8_t *keep, void *stream);
+/* The filter's reference importance ref [nabs] (pathfinder.py:266-271): that of the absorber's shortest two-leg path
+ * (paths ordered by slot, len [npath] their lengths; the first of equal ones), times its degeneracy if merged and the
+ * absorber has more than one candidate; 1 without paths. */
+int fm_find_ref(int32_t nabs, int64_t npath, const int32_t *slot, const float *len, const float *xport, const float *deg,
+                const int32_t *ncand, int32_t merged, float *ref, void *stream);
+/* The same filter as row numbers: pos[p] = the kept paths before p and *total their number, for npath <= 2^24
+ * (workspace of fm_scan_workspace_bytes(npath)); then the kept rows of paths of nleg legs, in order, with xport. */
+int fm_find_select(int64_t npath, const float *dtot, const float *xport, const int32_t *slot, const float *ref,
+                   float critpw, int64_t *pos, int64_t *total, void *workspace, size_t bytes, void *stream);
+int fm_find_compact(int64_t npath, int32_t nleg, const int64_t *pos, const int64_t *total, const fm_find_out *in,
+                    const float *xport, const fm_find_out *out, float *xport_out, void *stream);
 
 /* Launch policy (process-wide): the LDS in KiB (16..160) that a workgroup may take when the number of paths per
  * workgroup is chosen, for kernel 0 (FP32 forward calls), 1 (FP32 adjoints), 2 (FP64 forward), 3 (FP64 adjoints);
