@@ -90,3 +90,35 @@ def test_pieces_of_the_filter(critpw, monkeypatch):
     for bad in ([-1, 3], [len(pos)], torch.tensor([0, 10 ** 6], device="cuda")):
         with pytest.raises(ValueError, match="absorber index"):
             fd.enumerate_many(pos, float(box[0]), bad, ip)
+
+
+@pytest.mark.parametrize("npath", [1, 7, 32, 33])
+@pytest.mark.parametrize("nleg", range(2, 10))
+def test_importance_of_every_number_of_legs(nleg, npath):
+    """8 lanes per path, 32 paths per block. FP64 formula on the float32 tables and bins: a chain of up to 9 products and
+    divisions and an exponential per energy, 75 terms of one sign: 1e-5."""
+    from feffgpu_amd.pathfinder import GPUPathFinder, NBETA
+    fd = GPUPathFinder(str(GOLDEN / "validation" / "A018" / "phase.pad"))
+    rng = np.random.default_rng(10 * nleg + npath)
+    c = (rng.uniform(-3, 3, (npath, nleg, 3)) + 2.0 * np.arange(nleg)[None, :, None]).astype(np.float32)
+    c[:, 0] = 0
+    ip = rng.integers(0, fd.fbeta.shape[1], (npath, nleg))
+    got, rtot = (v.cpu().numpy() for v in fd._importance(c, ip))
+    leg = np.roll(c, -1, 1) - c
+    ri = np.sqrt((leg * leg).sum(-1))
+    u = leg / ri[..., None]
+    cosv = (u[:, :-1] * u[:, 1:]).sum(-1).astype(np.float32)
+    a = np.abs(cosv)
+    n = np.floor(a / np.float32(0.025))
+    n = (n + (a - n * np.float32(0.025) > np.float32(0.0125))) * np.where(cosv < 0, -1, 1)
+    k = np.clip(n.astype(int) + NBETA, 0, 2 * NBETA)
+    cmax = np.maximum(np.abs((u[:, -1] * u[:, 0]).sum(-1)), 0.3).astype(float)
+    fb, ck, xl, w = (v.double().cpu().numpy() for v in (fd.fbeta, fd.cksp, fd.xlam, fd.trap))
+    ri = ri.astype(float)
+    want = np.zeros(npath)
+    for i, e in enumerate(range(fd.ik0, len(ck))):
+        crit = cmax / (ri[:, -1] * ck[e])
+        for j in range(nleg - 1):
+            crit = crit * fb[e, ip[:, j + 1], k[:, j]] / (ri[:, j] * ck[e])
+        want += np.abs(crit * np.exp(-ri.sum(1) / xl[e])) * w[i]
+    assert np.allclose(got, want, rtol=1e-5, atol=0) and np.allclose(rtot, ri.sum(1), rtol=1e-6)
