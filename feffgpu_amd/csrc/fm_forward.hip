@@ -57,6 +57,8 @@ struct KArgs {
     size_t path_bytes;    // LDS per path of a workgroup
     unsigned *tickets;    // the path groups' counter pair of a persistent launch, or NULL (fixed assignment)
     void *keep;           // the bucket's kept scattering matrices (written), or NULL
+    uint32_t *rows;       // split launch: the output rows, path p's at rows + p row_words
+    size_t row_words;
 };
 
 int set_err(int code, const char *msg) {
@@ -69,7 +71,99 @@ int hip_err(hipError_t e, const char *where) {
 }
 
 
-template <class T, int SET>
+// ---- The split launch. The geometry of a path and its fine grid are chains of FP64 latencies with little parallelism,
+// which k_forward's two wavefronts per SIMD hide badly: of 1220 us (77 005 paths of 3 legs, K edge, FP32) they were 350
+// and 180. So k_rows fills a record per path (16 lanes each, seven wavefronts per SIMD) in the path's own row of the
+// output, k_forward reads the record and leaves cchi there, and k_fine turns it into chi(k): 904 us together (single
+// scattering, 32 828 paths: 244 -> 209; FP64, 12 838 paths of 3 legs: 468 -> 326). Below SPLIT_MIN paths the two more
+// launches cost more than that (700 paths of 3 legs 42 against 44 us, 1290 paths 66 against 56). Not for L and M edges
+// in FP32, whose kernel spills more so (51 213 paths of 3 legs, kept: 1268 against 1383 us).
+// A record: the leg lengths, cos/sin of eta and 2 eta, of beta and beta/2 (9 n doubles), R, reff, prod r, ok and the
+// potentials; after the bands the row holds cchi (2 E of T), reff (A) and ok. 32-bit words: rows need not be 8-byte
+// aligned.
+constexpr int SPLIT_MIN = 1280;
+template <class T, int SET> constexpr bool split_set() { return SET != 1 || sizeof(T) == 8; }
+__host__ __device__ constexpr int rec_words(int n) { return 2 * (9 * n + 3) + n + 1; }
+__device__ __forceinline__ void put_double(uint32_t *w, double v) { __builtin_memcpy(w, &v, 8); }
+__device__ __forceinline__ double get_double(const uint32_t *w) {
+    uint32_t x[2] = {w[0], w[1]};
+    double v;
+    __builtin_memcpy(&v, x, 8);
+    return v;
+}
+__global__ __launch_bounds__(256) void k_rows(KArgs a) {
+    __shared__ PathLDS gs[16];
+    const int t = threadIdx.x, n = a.nleg, lane = t & 15;
+    const int q = blockIdx.x * 16 + t / 16;
+    const int s0 = q < a.npath_bucket ? q : blockIdx.x * 16;
+    const int p = a.order ? a.order[a.first + s0] : a.first + s0;
+    PathLDS &g = gs[t / 16];
+    int ei;
+    load_path_group(a.src, p, g, ei, n, lane, true);
+    if (q >= a.npath_bucket) return;
+    uint32_t *const w = a.rows + (size_t)p * a.row_words;
+    if (lane < n) {
+        const int J = lane + 1;
+        const double v[9] = {g.r[J], g.c1[J], g.s1[J], g.c2[J], g.s2[J], g.cb[J], g.sb[J], g.ch[J], g.sh[J]};
+#pragma unroll
+        for (int f = 0; f < 9; ++f) put_double(w + 2 * (f * n + lane), v[f]);
+        w[2 * (9 * n + 3) + 1 + lane] = (uint32_t)g.ipot[lane];
+    }
+    if (lane == 0) {
+        put_double(w + 2 * (9 * n), g.R);
+        put_double(w + 2 * (9 * n + 1), g.reff);
+        put_double(w + 2 * (9 * n + 2), g.prod_r);
+        w[2 * (9 * n + 3)] = (uint32_t)g.ok;
+    }
+}
+// The record of path p into g, by one wavefront.
+__device__ __forceinline__ void load_record(const KArgs &a, int p, PathLDS &g, int lane) {
+    const int n = a.nleg;
+    const uint32_t *const w = a.rows + (size_t)p * a.row_words;
+    for (int x = lane; x < 9 * n; x += FM_WAVE) {
+        const int f = x / n, J = x - f * n + 1;
+        double *const to = f == 0 ? g.r : f < 5 ? g.c1 + (f - 1) * (FM_MAX_LEGS + 1) : g.cb + (f - 5) * (FM_MAX_LEGS + 1);
+        to[J] = get_double(w + 2 * x);
+    }
+    if (lane <= n) {
+        const uint32_t v = w[2 * (9 * n + 3) + lane];     // ok, then the potentials
+        if (lane == 0) { g.ok = (int)v; g.n = n; } else g.ipot[lane - 1] = (int)v;
+        if (lane == 1) g.ipot[n] = (int)v;
+    }
+    if (lane < 3) {
+        const double v = get_double(w + 2 * (9 * n + lane));
+        if (lane == 0) g.R = v; else if (lane == 1) g.reff = v; else g.prod_r = v;
+    }
+}
+// The fine grid of the paths whose rows hold cchi, one wavefront per path.
+template <class T> __global__ __launch_bounds__(FM_WAVE * 4) void k_fine(KArgs a, size_t wave_bytes) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int wid = threadIdx.x / FM_WAVE, lane = lane_id(), s0 = blockIdx.x * 4 + wid;
+    if (s0 >= a.npath_bucket) return;
+    const int p = a.order ? a.order[a.first + s0] : a.first + s0, E = a.ed.E, nk = a.G.nk;
+    T *const amp = reinterpret_cast<T *>(smem + (size_t)wid * wave_bytes);
+    double *const ang = reinterpret_cast<double *>(smem + (size_t)wid * wave_bytes + align16(sizeof(T) * (size_t)E));
+    uint32_t *const w = a.rows + (size_t)p * a.row_words;
+    T *const out = reinterpret_cast<T *>(w);
+    const uint32_t *const meta = w + 2 * E * (sizeof(T) / 4);
+    const double reff_A = get_double(meta);
+    if (meta[2]) {
+        for (int e = lane; e < E; e += FM_WAVE) {
+            const cx<T> c = mk<T>(out[2 * e], out[2 * e + 1]);
+            amp[e] = (T)sqrt((double)c.r * c.r + (double)c.i * c.i + 1e-30);
+            ang[e] = (double)atan2(c.i, c.r);
+        }
+        wave_sync();
+        fine_grid<T>(a.ed, a.G.jq + (size_t)a.edge_id * nk, a.G.fq + (size_t)a.edge_id * nk, a.G.q, nk, reff_A,
+                     a.src.P.sigma2 ? a.src.P.sigma2[p] : 0.0, amp, ang, out,
+                     a.G.S ? a.G.S + (size_t)a.edge_id * nk * a.G.sstride : nullptr, a.G.sstride);
+    } else {
+        for (int i = lane; i < nk; i += FM_WAVE) out[i] = (T)__builtin_nan("");
+    }
+}
+
+// SPLIT: of a split launch (the records of multiple-scattering paths read, cchi left in the rows of mode 1).
+template <class T, int SET, bool SPLIT = false>
 __global__ __launch_bounds__(FM_WAVE * 4) __attribute__((amdgpu_waves_per_eu(FM_WPE(T)))) void k_forward(KArgs a) {
     extern __shared__ __align__(16) unsigned char smem[];
     __shared__ int pidx[8], pval[8], tslot;
@@ -108,10 +202,15 @@ __global__ __launch_bounds__(FM_WAVE * 4) __attribute__((amdgpu_waves_per_eu(FM_
                 const int s0 = valid ? slot : blk * G;
                 const int p = a.order ? a.order[a.first + s0] : a.first + s0;
                 PathLDS &g = *reinterpret_cast<PathLDS *>(smem + (size_t)j * a.path_bytes);
-                int ei;
-                load_path(a.src, p, g, ei, nl);
+                if constexpr (SPLIT) {
+                    load_record(a, p, g, lane);
+                } else {
+                    int ei;
+                    load_path(a.src, p, g, ei, nl);
+                }
                 if (lane == 0) { pidx[j] = p; pval[j] = valid ? 1 : 0; }
             }
+            if constexpr (SPLIT) wave_sync();
         }
         if constexpr (SET < FM_SET_SS) build_tables<T, SET, false, 1>(ed, smem, a.path_bytes, off_W, 0, wid, 4, G, nl, ltab);
         __syncthreads();
@@ -139,6 +238,10 @@ __global__ __launch_bounds__(FM_WAVE * 4) __attribute__((amdgpu_waves_per_eu(FM_
                     T *o = reinterpret_cast<T *>(a.cchi_out) + ((size_t)pidx[jl] * E + e) * 2;
                     o[0] = gl.ok ? c.r : (T)__builtin_nan("");
                     o[1] = gl.ok ? c.i : (T)__builtin_nan("");
+                } else if constexpr (SPLIT) {
+                    T *const o = reinterpret_cast<T *>(a.rows + (size_t)pidx[jl] * a.row_words);
+                    o[2 * e] = c.r;
+                    o[2 * e + 1] = c.i;
                 } else {
                     T *amp = reinterpret_cast<T *>(lbase + off_amp);
                     double *ang = reinterpret_cast<double *>(lbase + off_ang);
@@ -156,7 +259,13 @@ __global__ __launch_bounds__(FM_WAVE * 4) __attribute__((amdgpu_waves_per_eu(FM_
             const int p = pidx[j];
             const double reff_A = g.ok ? g.reff * FM_BOHR : __builtin_nan("");
             if (lane == 0 && a.reff_out) a.reff_out[p] = reff_A;
-            if (a.src.mode == 1) {
+            if constexpr (SPLIT) {
+                if (a.src.mode == 1 && lane == 0) {
+                    uint32_t *const w = a.rows + (size_t)p * a.row_words + 2 * E * (sizeof(T) / 4);
+                    put_double(w, reff_A);
+                    w[2] = (uint32_t)g.ok;
+                }
+            } else if (a.src.mode == 1) {
                 const int nk = a.G.nk;
                 T *out = reinterpret_cast<T *>(a.chi_path) + (size_t)p * nk;
                 if (g.ok)
@@ -342,7 +451,7 @@ int set_for(const fm_edge &ed, int nleg) {
 
 // Paths per workgroup: the policy's, else the largest plan within the LDS budget (by default room for two workgroups
 // per CU), else the largest that fits one workgroup. Grid: one workgroup per group, or the policy's persistent grid.
-template <class T, int SET> hipError_t launch_forward(KArgs &a, const fm_launch &pol, hipStream_t st) {
+template <class T, int SET, bool SPLIT> hipError_t launch_main(KArgs &a, const fm_launch &pol, hipStream_t st) {
     const fm_edge &ed = a.ed;
     a.path_bytes = path_stride(align16(sizeof(PathLDS)) +
                                (SET < FM_SET_SS ? align16(sizeof(T) * rot_elems(a.nleg, ed.L1 + 1)) : 0) +
@@ -354,7 +463,7 @@ template <class T, int SET> hipError_t launch_forward(KArgs &a, const fm_launch 
     a.gp = 1 << g;
     a.bp = ed.bands[g];
     const size_t shm = a.path_bytes * a.gp;
-    const void *fn = (const void *)k_forward<T, SET>;
+    const void *fn = (const void *)k_forward<T, SET, SPLIT>;
     if (shm > 64 * 1024) {
         hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
         if (e != hipSuccess) return e;
@@ -364,8 +473,26 @@ template <class T, int SET> hipError_t launch_forward(KArgs &a, const fm_launch 
     if (e != hipSuccess) return e;
     if (blocks == 0) return hipSuccess;
     a.tickets = pol.grid != 0 ? pol.tickets : nullptr;
-    hipLaunchKernelGGL((k_forward<T, SET>), dim3((unsigned)blocks), dim3(FM_WAVE * 4), shm, st, a);
+    if (SPLIT && SET < FM_SET_SS)
+        hipLaunchKernelGGL(k_rows, dim3((unsigned)((a.npath_bucket + 15) / 16)), dim3(256), 0, st, a);
+    hipLaunchKernelGGL((k_forward<T, SET, SPLIT>), dim3((unsigned)blocks), dim3(FM_WAVE * 4), shm, st, a);
+    if (SPLIT && a.src.mode == 1) {
+        const size_t wb = align16(sizeof(T) * (size_t)ed.E) + align16(sizeof(double) * (size_t)ed.E);
+        hipLaunchKernelGGL(k_fine<T>, dim3((unsigned)((a.npath_bucket + 3) / 4)), dim3(FM_WAVE * 4), 4 * wb, st, a, wb);
+    }
     return hipGetLastError();
+}
+
+template <class T, int SET> hipError_t launch_forward(KArgs &a, const fm_launch &pol, hipStream_t st) {
+    // the split launch, where the output rows hold what it leaves there
+    const size_t cw = 2 * (size_t)a.ed.E * (sizeof(T) / 4);      // words of a path's cchi
+    a.rows = reinterpret_cast<uint32_t *>(a.src.mode == 1 ? a.chi_path : a.cchi_out);
+    a.row_words = a.src.mode == 1 ? (size_t)a.G.nk * (sizeof(T) / 4) : cw;
+    const size_t need = SET < FM_SET_SS ? (size_t)rec_words(a.nleg) : 0;
+    const bool fits = a.row_words >= need && (a.src.mode == 0 ? SET < FM_SET_SS : a.row_words >= cw + 3);
+    if constexpr (split_set<T, SET>())
+        if (a.npath_bucket > SPLIT_MIN && fits) return launch_main<T, SET, true>(a, pol, st);
+    return launch_main<T, SET, false>(a, pol, st);
 }
 
 template <class T, int SET> hipError_t launch_matrices(KArgs &a, const fm_launch &pol, hipStream_t st) {
