@@ -74,15 +74,14 @@ int hip_err(hipError_t e, const char *where) {
 // ---- The split launch. The geometry of a path and its fine grid are chains of FP64 latencies with little parallelism,
 // which k_forward's two wavefronts per SIMD hide badly: of 1220 us (77 005 paths of 3 legs, K edge, FP32) they were 350
 // and 180. So k_rows fills a record per path (16 lanes each, seven wavefronts per SIMD) in the path's own row of the
-// output, k_forward reads the record and leaves cchi there, and k_fine turns it into chi(k): 904 us together (single
-// scattering, 32 828 paths: 244 -> 209; FP64, 12 838 paths of 3 legs: 468 -> 326). Below SPLIT_MIN paths the two more
-// launches cost more than that (700 paths of 3 legs 42 against 44 us, 1290 paths 66 against 56). Not for L and M edges
-// in FP32, whose kernel spills more so (51 213 paths of 3 legs, kept: 1268 against 1383 us).
+// output, k_forward reads the record and leaves cchi there, and k_fine turns it into chi(k): 904 us together (L3 edge,
+// 51 213 paths of 3 legs: 1137 -> 765; single scattering, 32 828 paths: 244 -> 209; FP64, 12 838 paths of 3 legs: 468 ->
+// 326). Below SPLIT_MIN paths the two more launches cost more than that (700 paths of 3 legs 42 against 44 us, 1290 paths
+// 66 against 56).
 // A record: the leg lengths, cos/sin of eta and 2 eta, of beta and beta/2 (9 n doubles), R, reff, prod r, ok and the
 // potentials; after the bands the row holds cchi (2 E of T), reff (A) and ok. 32-bit words: rows need not be 8-byte
 // aligned.
 constexpr int SPLIT_MIN = 1280;
-template <class T, int SET> constexpr bool split_set() { return SET != 1 || sizeof(T) == 8; }
 __host__ __device__ constexpr int rec_words(int n) { return 2 * (9 * n + 3) + n + 1; }
 __device__ __forceinline__ void put_double(uint32_t *w, double v) { __builtin_memcpy(w, &v, 8); }
 __device__ __forceinline__ double get_double(const uint32_t *w) {
@@ -490,8 +489,7 @@ template <class T, int SET> hipError_t launch_forward(KArgs &a, const fm_launch 
     a.row_words = a.src.mode == 1 ? (size_t)a.G.nk * (sizeof(T) / 4) : cw;
     const size_t need = SET < FM_SET_SS ? (size_t)rec_words(a.nleg) : 0;
     const bool fits = a.row_words >= need && (a.src.mode == 0 ? SET < FM_SET_SS : a.row_words >= cw + 3);
-    if constexpr (split_set<T, SET>())
-        if (a.npath_bucket > SPLIT_MIN && fits) return launch_main<T, SET, true>(a, pol, st);
+    if (a.npath_bucket > SPLIT_MIN && fits) return launch_main<T, SET, true>(a, pol, st);
     return launch_main<T, SET, false>(a, pol, st);
 }
 

@@ -608,9 +608,10 @@ __device__ __forceinline__ void keep_load(const T *b, int E, cx<T> (&Ft)[FM_NREP
     }
 }
 
-// keep: the lane's pointer into the kept scattering matrices (written after each is built), or NULL.
+// keep: the lane's pointer into the kept scattering matrices (written after each is built), or NULL. Inlined into each
+// of its kernels: called out of line it cost an L3 list 30% (its arrays in scratch memory).
 template <class T, int SET>
-__device__ cx<T> path_cchi(const fm_edge &ed, const PathLDS &g, const T *W, int ltab, int e, int n, T *keep = nullptr) {
+__device__ __forceinline__ cx<T> path_cchi(const fm_edge &ed, const PathLDS &g, const T *W, int ltab, int e, int n, T *keep = nullptr) {
     constexpr LamDef D = lamdef(SET);
     constexpr PairDef PD = pairdef(SET);
     constexpr int L = D.L, L0 = D.L0;
