@@ -155,6 +155,12 @@ def lib():
                                             ctypes.POINTER(_i32), ctypes.POINTER(_i32), ctypes.POINTER(_i32), _vp, _vp,
                                             _vp, _i32, _vp, _vp, _vp, _vp, _vp, ctypes.c_size_t,
                                             ctypes.POINTER(FmLaunch), _vp]
+        L.fm_chi_paths_overlap.argtypes = L.fm_chi_paths.argtypes[:-1] + [_vp, _vp]
+        L.fm_chi_paths_backward_overlap.argtypes = L.fm_chi_paths_backward.argtypes[:-1] + [_vp, _vp]
+        L.fm_backward_overlap_bytes.restype = _sz
+        L.fm_backward_overlap_bytes.argtypes = [_i32, ctypes.POINTER(FmEdge), _i32] + [ctypes.POINTER(_i32)] * 3 + [_i32]
+        L.fm_overlap_acquire.restype = _vp
+        L.fm_overlap_release.argtypes = [_vp]
         L.fm_plain_path_bytes.restype = ctypes.c_size_t
         L.fm_keep_bytes.restype = ctypes.c_size_t
         L.fm_keep_bytes.argtypes = [_i32, ctypes.POINTER(FmEdge), _i32, _i32]
@@ -194,11 +200,11 @@ def ptr(t) -> int | None:
 
 
 def backward_workspace(precision: int, nlegmax: int, npath: int, device, E: int, max_slots: int = 4096,
-                       max_region_bytes: int = 2 << 30):
+                       max_region_bytes: int = 2 << 30, at_least: int = 0):
     """A device buffer for the adjoints: paths of 7-9 legs, band slots for the workgroups in flight (a workgroup takes
     one per band of its plan, at most 16), at most max_slots and no more than npath workgroups need; paths of 2-6 legs,
     for each of up to npath paths of a launch the chain's matrices, the scattering matrices and cchi of an adjoint whose
-    forward kept none, and a record, at most max_region_bytes (larger buckets run in chunks)."""
+    forward kept none, and a record, at most max_region_bytes (larger buckets run in chunks); at_least bytes."""
     slots = max(16, min(int(max_slots), 16 * max(int(npath), 1))) if nlegmax > 6 else 16
     nbytes = lib().fm_backward_workspace_bytes(int(precision), int(nlegmax), slots)
     n, ec = min(int(nlegmax), 6), 8 if precision == 32 else 16
@@ -206,7 +212,7 @@ def backward_workspace(precision: int, nlegmax: int, npath: int, device, E: int,
     if n > 2:
         per = max(per, (40 * (n - 1) + n + 4) * (int(E) + 3) * ec + 8 * (10 * n + 5) + ec // 2 * (4 * n + 160))
     nbytes = max(nbytes, min((int(npath) + 32) * per, int(max_region_bytes)))
-    return torch.empty(max(nbytes, 1), dtype=torch.uint8, device=device)
+    return torch.empty(max(nbytes, int(at_least), 1), dtype=torch.uint8, device=device)
 
 
 def stream_of(device) -> int:

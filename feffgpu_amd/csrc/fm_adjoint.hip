@@ -1117,6 +1117,14 @@ template <class T> hipError_t launch_ms(const MsAdjoint &m, const fm_launch &pol
 
 namespace fm {
 
+size_t ms_adjoint_bytes(int precision, const fm_edge &ed, int nleg, int cnt, bool keep) {
+    const size_t es = precision == 32 ? 4 : 8;
+    const size_t rows = ed.ilinit <= 1 ? keep_rows<0>(nleg) : keep_rows<1>(nleg);
+    const size_t path = sizeof(double) * rec_len(nleg) + es * rt_len(nleg) + slot_rows(nleg) * (size_t)ed.E * 2 * es +
+                        (keep ? 0 : rows * ed.E * 2 * es);
+    return (size_t)((cnt + KG - 1) / KG) * (k_group((int)rows, ed.E) * 2 * es + KG * path) + 2048;
+}
+
 size_t ms_adjoint_bytes16(int precision, int nleg) {
     const size_t ec = precision == 32 ? 8 : 16;
     const size_t rows = keep_rows<1>(nleg) > keep_rows<0>(nleg) ? keep_rows<1>(nleg) : keep_rows<0>(nleg);

@@ -1212,6 +1212,28 @@ int scratch_of_current_device(void **out) {
     return FM_OK;
 }
 
+// The workspace region of every lane: what its largest bucket runs in without chunks; returns their sum, 0 if a bucket
+// is of more legs than the multiple-scattering adjoint takes (its workgroups fill any workspace).
+template <class Kept>
+size_t lane_regions(int precision, const fm_edge *edges, int nbucket, const int32_t *offset, const int32_t *edge,
+                    const int32_t *nleg, Kept kept, const std::vector<int> &lane, size_t *region) {
+    for (int i = 0; i <= FM_SIDE; ++i) region[i] = 0;
+    for (int b = 0; b < nbucket; ++b) {
+        const int cnt = offset[b + 1] - offset[b];
+        if (cnt <= 0) continue;
+        if (nleg[b] > FM_FUSED_MAXLEG) return 0;
+        const fm_edge &ed = edges[edge ? edge[b] : 0];
+        size_t need = (size_t)(cnt + 1) * 9 * ed.E * (precision == 32 ? 8 : 16);
+        if (nleg[b] > 2) need = ms_adjoint_bytes(precision, ed, nleg[b], cnt, kept(b));
+        else if (need > FM_DREGION_MAX) need = FM_DREGION_MAX;
+        need = (need + 255) & ~size_t(255);
+        if (need > region[lane[b]]) region[lane[b]] = need;
+    }
+    size_t sum = 0;
+    for (int i = 0; i <= FM_SIDE; ++i) sum += region[i];
+    return sum;
+}
+
 }  // namespace
 
 extern "C" {
@@ -1326,9 +1348,33 @@ int fm_chi_fine_backward(const fm_edge *edge, int32_t precision, int32_t npath, 
 int fm_chi_paths_backward(const fm_edge *edges, int32_t nedge, const fm_paths *paths, const fm_grid *grid,
                           int32_t precision, int32_t iorder, const int32_t *order, int32_t nbucket,
                           const int32_t *bucket_offset, const int32_t *bucket_kind, const int32_t *bucket_edge,
-                          const int32_t *bucket_nleg, const int32_t *segment, const double *gseg, const void *gpath, int32_t natom,
-                          const int32_t *atom_ptr, const int32_t *atom_refs, double *gcoord, double *grad_pos,
-                          void *workspace, size_t workspace_bytes, const fm_launch *launch, void *stream) {
+                          const int32_t *bucket_nleg, const int32_t *segment, const double *gseg, const void *gpath,
+                          int32_t natom, const int32_t *atom_ptr, const int32_t *atom_refs, double *gcoord,
+                          double *grad_pos, void *workspace, size_t workspace_bytes, const fm_launch *launch,
+                          void *stream) {
+    return fm_chi_paths_backward_overlap(edges, nedge, paths, grid, precision, iorder, order, nbucket, bucket_offset,
+                                         bucket_kind, bucket_edge, bucket_nleg, segment, gseg, gpath, natom, atom_ptr,
+                                         atom_refs, gcoord, grad_pos, workspace, workspace_bytes, launch, nullptr, stream);
+}
+
+size_t fm_backward_overlap_bytes(int32_t precision, const fm_edge *edges, int32_t nbucket, const int32_t *bucket_offset,
+                                 const int32_t *bucket_edge, const int32_t *bucket_nleg, int32_t kept) try {
+    if (!edges || nbucket < 1 || !bucket_offset || !bucket_nleg || (precision != 32 && precision != 64)) return 0;
+    const std::vector<int> lane = lanes_of(nbucket, bucket_offset, bucket_nleg, 1 + FM_SIDE);
+    size_t region[1 + FM_SIDE];
+    return lane_regions(precision, edges, nbucket, bucket_offset, bucket_edge, bucket_nleg,
+                        [&](int) { return kept != 0; }, lane, region);
+} catch (const std::exception &) {
+    return 0;
+}
+
+int fm_chi_paths_backward_overlap(const fm_edge *edges, int32_t nedge, const fm_paths *paths, const fm_grid *grid,
+                                  int32_t precision, int32_t iorder, const int32_t *order, int32_t nbucket,
+                                  const int32_t *bucket_offset, const int32_t *bucket_kind, const int32_t *bucket_edge,
+                                  const int32_t *bucket_nleg, const int32_t *segment, const double *gseg,
+                                  const void *gpath, int32_t natom, const int32_t *atom_ptr, const int32_t *atom_refs,
+                                  double *gcoord, double *grad_pos, void *workspace, size_t workspace_bytes,
+                                  const fm_launch *launch, fm_overlap *overlap, void *stream) try {
     if (nedge < 1 || nedge > FM_MAX_EDGE) return set_err(FM_EINVAL, "nedge out of range 1..4");
     int emax = 0;
     for (int i = 0; i < nedge; ++i) {
@@ -1350,6 +1396,32 @@ int fm_chi_paths_backward(const fm_edge *edges, int32_t nedge, const fm_paths *p
         return set_err(FM_EINVAL, "workspace smaller than fm_backward_workspace_bytes(precision, nmax, 16)");
     if (nbucket > 0 && (!bucket_offset || !bucket_kind || !bucket_nleg)) return set_err(FM_EINVAL, "NULL bucket arrays");
     hipStream_t st = (hipStream_t)stream;
+    // the buckets of different lanes run at the same time, so each lane has a region of the workspace; if it does not
+    // hold them all, one lane has it whole
+    std::vector<int> lane(nbucket > 0 ? nbucket : 0, 0);
+    size_t region[1 + FM_SIDE] = {workspace_bytes};
+    int want = 1;
+    if (overlap && nbucket > 1) {
+        bool valid = true;      // what the loop below refuses is left to it
+        for (int b = 0; b < nbucket; ++b)
+            valid = valid && bucket_nleg[b] >= 2 && bucket_nleg[b] <= FM_MAX_LEGS &&
+                    (!bucket_edge || (bucket_edge[b] >= 0 && bucket_edge[b] < nedge));
+        size_t r[1 + FM_SIDE];
+        if (valid) {
+            std::vector<int> l = lanes_of(nbucket, bucket_offset, bucket_nleg, 1 + FM_SIDE);
+            const size_t all = lane_regions(precision, edges, nbucket, bucket_offset, bucket_edge, bucket_nleg,
+                                            [&](int b) { return launch && launch[b].keep; }, l, r);
+            if (all != 0 && all <= workspace_bytes) {
+                want = nbucket;
+                lane.swap(l);
+                memcpy(region, r, sizeof region);
+            }
+        }
+    }
+    Lanes lanes(overlap, st, want);
+    unsigned char *start[1 + FM_SIDE];
+    start[0] = (unsigned char *)workspace;
+    for (int i = 1; i <= FM_SIDE; ++i) start[i] = start[i - 1] + (want > 1 ? region[i - 1] : 0);
     for (int b = 0; b < nbucket; ++b) {
         const int cnt = bucket_offset[b + 1] - bucket_offset[b];
         if (cnt <= 0) continue;
@@ -1379,8 +1451,8 @@ int fm_chi_paths_backward(const fm_edge *edges, int32_t nedge, const fm_paths *p
         if ((kind == FM_BUCKET_K_MS) != (a.ed.ilinit <= 1) && kind != FM_BUCKET_SS)
             return set_err(FM_EINVAL, "bucket kind does not match its edge");
         const int set = set_of(a.ed, a.nlegmax);
-        a.work = (unsigned char *)workspace;
-        a.work_bytes = workspace_bytes;
+        a.work = start[lane[b]];
+        a.work_bytes = region[lane[b]];
         const fm_launch pol = policy_of_b(launch, b);
         if (pol.gpaths != 0 && pol.gpaths != 1 && pol.gpaths != 2 && pol.gpaths != 4 && pol.gpaths != 8)
             return set_err(FM_EINVAL, "launch policy: gpaths must be 0, 1, 2, 4 or 8");
@@ -1390,7 +1462,8 @@ int fm_chi_paths_backward(const fm_edge *edges, int32_t nedge, const fm_paths *p
                 return set_err(FM_EINVAL, "fm_chi_paths_backward: keep_bytes smaller than fm_keep_bytes for the bucket");
             a.keep = pol.keep;
         }
-        hipError_t e = precision == 32 ? dispatch_b<float>(a, set, pol, st) : dispatch_b<double>(a, set, pol, st);
+        hipError_t e = precision == 32 ? dispatch_b<float>(a, set, pol, lanes.at(lane[b]))
+                                        : dispatch_b<double>(a, set, pol, lanes.at(lane[b]));
         if (e == hipErrorInvalidValue)
             return set_err(FM_EINVAL, "fm_chi_paths_backward: the bucket's paths do not fit one workgroup's LDS");
         if (e == hipErrorInvalidConfiguration)
@@ -1399,6 +1472,7 @@ int fm_chi_paths_backward(const fm_edge *edges, int32_t nedge, const fm_paths *p
         if (e == hipErrorOutOfMemory) return set_err(FM_EINVAL, "fm_chi_paths_backward: workspace too small for one path");
         if (e != hipSuccess) return hip_err(e, "fm_chi_paths_backward launch");
     }
+    if (hipError_t e = lanes.join()) return hip_err(e, "fm_chi_paths_backward side streams");
     if (grad_pos && natom > 0) {
         if (!atom_ptr || !atom_refs) return set_err(FM_EINVAL, "NULL atom lists");
         hipLaunchKernelGGL(k_atom_grad, dim3((natom + 3) / 4), dim3(FM_WAVE * 4), 0, st, natom, atom_ptr, atom_refs,
@@ -1407,6 +1481,8 @@ int fm_chi_paths_backward(const fm_edge *edges, int32_t nedge, const fm_paths *p
         if (e != hipSuccess) return hip_err(e, "atom gradient launch");
     }
     return FM_OK;
+} catch (const std::exception &) {
+    return set_err(FM_EINVAL, "fm_chi_paths_backward: out of host memory");
 }
 
 }  // extern "C"

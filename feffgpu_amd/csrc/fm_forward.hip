@@ -644,11 +644,22 @@ int fm_chi_fine(const fm_edge *edge, int32_t precision, int32_t npath, const voi
     return e == hipSuccess ? FM_OK : hip_err(e, "fm_chi_fine launch");
 }
 
-int fm_chi_paths(const fm_edge *edges, int32_t nedge, const fm_paths *paths, const fm_grid *grid,
+int fm_chi_paths(const fm_edge *edges, int32_t nedge, const fm_paths *paths, const fm_grid *grid, int32_t precision,
+                 int32_t iorder, const int32_t *order, int32_t nbucket, const int32_t *bucket_offset,
+                 const int32_t *bucket_kind, const int32_t *bucket_edge, const int32_t *bucket_nleg, int32_t nseg,
+                 const int32_t *seg_ptr, const int32_t *seg_paths, double *chi_seg, void *chi_path, double *reff,
+                 const fm_launch *launch, void *stream) {
+    return fm_chi_paths_overlap(edges, nedge, paths, grid, precision, iorder, order, nbucket, bucket_offset, bucket_kind,
+                                bucket_edge, bucket_nleg, nseg, seg_ptr, seg_paths, chi_seg, chi_path, reff, launch,
+                                nullptr, stream);
+}
+
+int fm_chi_paths_overlap(const fm_edge *edges, int32_t nedge, const fm_paths *paths, const fm_grid *grid,
                          int32_t precision, int32_t iorder, const int32_t *order, int32_t nbucket,
                          const int32_t *bucket_offset, const int32_t *bucket_set, const int32_t *bucket_edge,
-                         const int32_t *bucket_nleg, int32_t nseg, const int32_t *seg_ptr, const int32_t *seg_paths, double *chi_seg,
-                         void *chi_path, double *reff, const fm_launch *launch, void *stream) {
+                         const int32_t *bucket_nleg, int32_t nseg, const int32_t *seg_ptr, const int32_t *seg_paths,
+                         double *chi_seg, void *chi_path, double *reff, const fm_launch *launch, fm_overlap *overlap,
+                         void *stream) try {
     if (nedge < 1 || nedge > FM_MAX_EDGE) return set_err(FM_EINVAL, "nedge out of range 1..4");
     for (int i = 0; i < nedge; ++i) {
         int rc = check_edge(&edges[i]);
@@ -663,6 +674,8 @@ int fm_chi_paths(const fm_edge *edges, int32_t nedge, const fm_paths *paths, con
         if (grid->S && grid->sstride < edges[i].E) return set_err(FM_EINVAL, "grid.sstride < E");
     if (nbucket > 0 && (!bucket_offset || !bucket_set || !bucket_nleg)) return set_err(FM_EINVAL, "NULL bucket arrays");
     hipStream_t st = (hipStream_t)stream;
+    Lanes lanes(overlap, st, nbucket);
+    const std::vector<int> lane = lanes_of(nbucket, bucket_offset, bucket_nleg, lanes.n);
     for (int b = 0; b < nbucket; ++b) {
         const int cnt = bucket_offset[b + 1] - bucket_offset[b];
         if (cnt <= 0) continue;
@@ -694,12 +707,14 @@ int fm_chi_paths(const fm_edge *edges, int32_t nedge, const fm_paths *paths, con
                 return set_err(FM_EINVAL, "fm_chi_paths: keep_bytes smaller than fm_keep_bytes for the bucket");
             a.keep = pol.keep;
         }
-        hipError_t e = precision == 32 ? dispatch<float>(a, set, pol, st) : dispatch<double>(a, set, pol, st);
+        hipError_t e = precision == 32 ? dispatch<float>(a, set, pol, lanes.at(lane[b]))
+                                        : dispatch<double>(a, set, pol, lanes.at(lane[b]));
         if (e == hipErrorInvalidValue) return set_err(FM_EINVAL, "fm_chi_paths: the bucket's paths do not fit one workgroup's LDS");
         if (e == hipErrorInvalidConfiguration)
             return set_err(FM_EINVAL, "fm_chi_paths: the launch policy's gpaths has no band plan or does not fit one CU's LDS");
         if (e != hipSuccess) return hip_err(e, "fm_chi_paths launch");
     }
+    if (hipError_t e = lanes.join()) return hip_err(e, "fm_chi_paths side streams");
     if (chi_seg && nseg > 0) {
         if (!seg_ptr || !seg_paths) return set_err(FM_EINVAL, "NULL segment lists");
         dim3 grd((grid->nk + FM_WAVE - 1) / FM_WAVE, nseg);
@@ -713,6 +728,8 @@ int fm_chi_paths(const fm_edge *edges, int32_t nedge, const fm_paths *paths, con
         if (e != hipSuccess) return hip_err(e, "segment sum launch");
     }
     return FM_OK;
+} catch (const std::exception &) {
+    return set_err(FM_EINVAL, "fm_chi_paths: out of host memory");
 }
 
 }  // extern "C"

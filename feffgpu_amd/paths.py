@@ -18,6 +18,7 @@ from __future__ import annotations
 from dataclasses import dataclass
 
 import ctypes
+import weakref
 
 import numpy as np
 import torch
@@ -25,6 +26,8 @@ import torch
 from . import _native as N
 from .pad import load_phase
 from .tables import edge_tables, energies_needed, interpolation, spline_matrix
+
+OVERLAP_BYTES = 4 << 30    # the largest adjoint workspace for buckets that run next to each other
 
 
 def _cell_struct(cell):
@@ -213,8 +216,6 @@ class PathPlan:
         self.atom_ptr_t = i32(np.cumsum(ptr))
         self.atom_refs_t = i32(ref_id[o])
         self.gcoord = torch.empty(Pn, nmax, 3, dtype=torch.float64, device=dev)
-        big = int(np.diff(self.buckets.offset).max()) if Pn else 0
-        self.workspace = N.backward_workspace(self.precision, nmax, big, dev, max(T.E for T in self.tables)) if Pn else None
         self.chi_path = torch.empty(Pn, nk, dtype=self.rdtype, device=dev)
         self.reff = torch.empty(Pn, dtype=torch.float64, device=dev)
         self._h_off = (N._i32 * len(self.buckets.offset))(*self.buckets.offset.tolist())
@@ -223,6 +224,20 @@ class PathPlan:
         self._h_nlm = (N._i32 * max(1, len(self.buckets.nleg)))(*self.buckets.nleg.tolist())
         if self.keep_amplitudes and self.keep_bytes() > self.keep_limit_bytes:
             self.keep_amplitudes = False
+        # several buckets run next to each other on side streams (this plan's alone, back to the library's pool with
+        # it); the adjoint needs a workspace region for each of them then
+        nbk = len(self.buckets.kind)
+        self._overlap, beside = None, 0
+        if nbk > 1:
+            with torch.cuda.device(dev):
+                self._overlap = N.lib().fm_overlap_acquire()
+            if self._overlap:
+                weakref.finalize(self, N.lib().fm_overlap_release, self._overlap).atexit = False
+                beside = int(N.lib().fm_backward_overlap_bytes(self.precision, self.edge_array, nbk, self._h_off,
+                                                               self._h_edge, self._h_nlm, int(self.keep_amplitudes)))
+        big = int(np.diff(self.buckets.offset).max()) if Pn else 0
+        self.workspace = N.backward_workspace(self.precision, nmax, big, dev, max(T.E for T in self.tables),
+                                              at_least=beside if beside <= OVERLAP_BYTES else 0) if Pn else None
         # per-bucket launch policies of the forward (0) and adjoint (1) calls: defaults until set_launch / tune;
         # every bucket and kernel has its own zeroed counter pair for persistent launches that take groups in turn
         nb = max(1, len(self.buckets.kind))
@@ -322,11 +337,12 @@ class PathPlan:
         chi_seg = torch.empty(self.nseg, self.nk, dtype=torch.float64, device=self.device) if want_seg else None
         if self.npath:
             ps = self._paths_struct(pos64)
-            N.check(N.lib().fm_chi_paths(self.edge_array, len(self.edges), ps, self.grid, self.precision, self.iorder,
-                                         self.order_t.data_ptr(), len(self.buckets.kind), self._h_off, self._h_kind,
-                                         self._h_edge, self._h_nlm, self.nseg, self.seg_ptr_t.data_ptr(), self.seg_paths_t.data_ptr(),
-                                         N.ptr(chi_seg), self.chi_path.data_ptr(), self.reff.data_ptr(),
-                                         self._policy(0, keep=keep), N.stream_of(self.device)), "fm_chi_paths")
+            N.check(N.lib().fm_chi_paths_overlap(
+                self.edge_array, len(self.edges), ps, self.grid, self.precision, self.iorder, self.order_t.data_ptr(),
+                len(self.buckets.kind), self._h_off, self._h_kind, self._h_edge, self._h_nlm, self.nseg,
+                self.seg_ptr_t.data_ptr(), self.seg_paths_t.data_ptr(), N.ptr(chi_seg), self.chi_path.data_ptr(),
+                self.reff.data_ptr(), self._policy(0, keep=keep), self._overlap, N.stream_of(self.device)),
+                "fm_chi_paths")
             if keep:
                 self.kept_generation += 1
         elif want_seg:
@@ -351,14 +367,13 @@ class PathPlan:
         if gp is not None and tuple(gp.shape) != (self.npath, self.nk):
             raise ValueError("gpath must be (P, NK)")
         ps = self._paths_struct(pos64)
-        N.check(N.lib().fm_chi_paths_backward(self.edge_array, len(self.edges), ps, self.grid, self.precision,
-                                              self.iorder, self.order_t.data_ptr(), len(self.buckets.kind), self._h_off,
-                                              self._h_kind, self._h_edge, self._h_nlm, self.segment_t.data_ptr(), N.ptr(gs),
-                                              N.ptr(gp), self.natom_ref, self.atom_ptr_t.data_ptr(),
-                                              self.atom_refs_t.data_ptr(), self.gcoord.data_ptr(), grad.data_ptr(),
-                                              self.workspace.data_ptr(), self.workspace.numel(),
-                                              self._policy(1, keep=kept and self._keep is not None),
-                                              N.stream_of(self.device)), "fm_chi_paths_backward")
+        N.check(N.lib().fm_chi_paths_backward_overlap(
+            self.edge_array, len(self.edges), ps, self.grid, self.precision, self.iorder, self.order_t.data_ptr(),
+            len(self.buckets.kind), self._h_off, self._h_kind, self._h_edge, self._h_nlm, self.segment_t.data_ptr(),
+            N.ptr(gs), N.ptr(gp), self.natom_ref, self.atom_ptr_t.data_ptr(), self.atom_refs_t.data_ptr(),
+            self.gcoord.data_ptr(), grad.data_ptr(), self.workspace.data_ptr(), self.workspace.numel(),
+            self._policy(1, keep=kept and self._keep is not None), self._overlap, N.stream_of(self.device)),
+            "fm_chi_paths_backward")
         return grad
 
     def __call__(self, pos):

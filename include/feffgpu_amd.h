@@ -207,6 +207,32 @@ int fm_chi_paths_backward(const fm_edge *edges, int32_t nedge, const fm_paths *p
                           const int32_t *atom_ptr, const int32_t *atom_refs, double *gcoord, double *grad_pos,
                           void *workspace, size_t workspace_bytes, const fm_launch *launch, void *stream);
 
+/* The same calls with the buckets running next to each other on the call's stream and two side streams of `overlap`
+ * (NULL: one after the other, as above). The side streams wait for the stream at the start of the call and the stream
+ * for them at its end, also under capture. The adjoint gives every lane a region of the workspace if it holds at least
+ * fm_backward_overlap_bytes (kept: the launches carry kept matrices; 0: buckets of more than 6 legs, which do not
+ * overlap), and runs the buckets one after the other if not. A set belongs to the device that was current when it was
+ * acquired and to one caller at a time (calls that use the same set must not run at the same time); released sets are
+ * kept for the next caller, a few per device. */
+typedef struct fm_overlap fm_overlap;
+fm_overlap *fm_overlap_acquire(void);
+void fm_overlap_release(fm_overlap *overlap);
+int fm_chi_paths_overlap(const fm_edge *edges, int32_t nedge, const fm_paths *paths, const fm_grid *grid,
+                         int32_t precision, int32_t iorder, const int32_t *order, int32_t nbucket,
+                         const int32_t *bucket_offset, const int32_t *bucket_kind, const int32_t *bucket_edge,
+                         const int32_t *bucket_nleg, int32_t nseg, const int32_t *seg_ptr, const int32_t *seg_paths,
+                         double *chi_seg, void *chi_path, double *reff, const fm_launch *launch, fm_overlap *overlap,
+                         void *stream);
+size_t fm_backward_overlap_bytes(int32_t precision, const fm_edge *edges, int32_t nbucket, const int32_t *bucket_offset,
+                                 const int32_t *bucket_edge, const int32_t *bucket_nleg, int32_t kept);
+int fm_chi_paths_backward_overlap(const fm_edge *edges, int32_t nedge, const fm_paths *paths, const fm_grid *grid,
+                                  int32_t precision, int32_t iorder, const int32_t *order, int32_t nbucket,
+                                  const int32_t *bucket_offset, const int32_t *bucket_kind, const int32_t *bucket_edge,
+                                  const int32_t *bucket_nleg, const int32_t *segment, const double *gseg,
+                                  const void *gpath, int32_t natom, const int32_t *atom_ptr, const int32_t *atom_refs,
+                                  double *gcoord, double *grad_pos, void *workspace, size_t workspace_bytes,
+                                  const fm_launch *launch, fm_overlap *overlap, void *stream);
+
 /* The plain FP64 path stage: the reference's op sequence (src/feffgpu/stage.py:147-388) with one kernel per stage
  * and every intermediate (rotation matrices, spherical-wave factors, gam / gamtl, scattering matrices, termination,
  * cchi) in HBM -- the comparator of the fused kernels on the same GPU, and an independent evaluation for tests.
