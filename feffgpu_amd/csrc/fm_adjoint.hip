@@ -989,6 +989,10 @@ constexpr size_t ST_STATIC = sizeof(StreamUnit) * ST_MAXU + sizeof(double) * 12 
 template <class T, int SET, int NL> hipError_t launch_nl(const MsAdjoint &m, MArgs<T> &a, long room, const fm_launch &pol,
                                                          hipStream_t st) {
     constexpr int WPE = sizeof(T) == 4 ? 2 : 1;
+    // k_chain: two wavefronts per SIMD where its matrices fit 256 registers (K edge, 3 legs: 244), else one with 512: the
+    // spills cost more than the second wavefront hides (FP32, us, two / one: L3 edge, 4 legs, 38 967 paths 1988 / 1007,
+    // 5 legs, 16 291 paths 1262 / 683; K edge, 4 legs, 36 909 paths 692 / 663, 5 legs, 15 111 paths 547 / 415)
+    constexpr int CWPE = sizeof(T) == 4 && SET == 0 && NL <= 3 ? 2 : 1;
     constexpr int rows = keep_rows<SET>(NL);
     const fm_edge &ed = m.ed;
     const int E = ed.E;
@@ -1047,7 +1051,7 @@ template <class T, int SET, int NL> hipError_t launch_nl(const MsAdjoint &m, MAr
             a.F = fw;
         }
         hipLaunchKernelGGL((k_setup<T, SET>), dim3((unsigned)((cnt + 15) / 16)), dim3(256), 0, st, a);
-        hipLaunchKernelGGL((k_chain<T, SET, NL, WPE>), dim3((unsigned)(((long)cnt * nchunk + 3) / 4)), dim3(FM_WAVE * 4), 0, st, a);
+        hipLaunchKernelGGL((k_chain<T, SET, NL, CWPE>), dim3((unsigned)(((long)cnt * nchunk + 3) / 4)), dim3(FM_WAVE * 4), 0, st, a);
         hipLaunchKernelGGL((k_pbc<T, NL>), dim3((unsigned)((cnt + 3) / 4)), dim3(FM_WAVE * 4), shm_c, st, a);
         // units per workgroup: 16 (bands of 4 energies, the most even), halved while the LDS does not hold them or the
         // launch would leave CUs without work (down to 4, whose four bands are one wavefront's each)

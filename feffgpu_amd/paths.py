@@ -27,7 +27,7 @@ from . import _native as N
 from .pad import load_phase
 from .tables import edge_tables, energies_needed, interpolation, spline_matrix
 
-OVERLAP_BYTES = 4 << 30    # the largest adjoint workspace for buckets that run next to each other
+OVERLAP_BYTES = 8 << 30    # the largest adjoint workspace for buckets that run next to each other
 
 
 def _cell_struct(cell):
