@@ -115,23 +115,50 @@ __global__ __launch_bounds__(256) void k_rows(KArgs a) {
         w[2 * (9 * n + 3)] = (uint32_t)g.ok;
     }
 }
-// The record of path p into g, by one wavefront.
-__device__ __forceinline__ void load_record(const KArgs &a, int p, PathLDS &g, int lane) {
-    const int n = a.nleg;
-    const uint32_t *const w = a.rows + (size_t)p * a.row_words;
-    for (int x = lane; x < 9 * n; x += FM_WAVE) {
-        const int f = x / n, J = x - f * n + 1;
+// The records of the wavefront's paths j = wid, wid + 4, ... < G of group blk (np <= 2) into LDS, their numbers into
+// pidx and pval: every lane fetches its own path's number and item, so that both latencies are waited for once.
+__device__ __forceinline__ void load_records(const KArgs &a, int blk, int G, int wid, int lane, unsigned char *smem, int *pidx,
+                                             int *pval) {
+    const int n = a.nleg, np = wid < G ? (G - 1 - wid) / 4 + 1 : 0;
+    auto path = [&](int j, bool &valid) {
+        const int slot = blk * G + j;
+        valid = slot < a.npath_bucket;
+        const int s0 = valid ? slot : blk * G;
+        return a.order ? a.order[a.first + s0] : a.first + s0;
+    };
+    // R, reff, prod r; ok and the potentials
+    const int q = lane / (n + 4), k = lane - q * (n + 4), j = wid + 4 * (q < np ? q : 0);
+    bool valid;
+    const int p = path(j < G ? j : 0, valid);
+    const uint32_t *const w = a.rows + (size_t)p * a.row_words + 2 * 9 * n;
+    double d = 0.0;
+    uint32_t v = 0;
+    if (k < 3) d = get_double(w + 2 * k); else v = w[6 + k - 3];
+    for (int x = lane; x < np * 9 * n; x += FM_WAVE) {
+        const int xq = x / (9 * n), i = x - xq * 9 * n, f = i / n, J = i - f * n + 1, xj = wid + 4 * xq;
+        bool xv;
+        const double t = get_double(a.rows + (size_t)path(xj, xv) * a.row_words + 2 * i);
+        PathLDS &g = *reinterpret_cast<PathLDS *>(smem + (size_t)xj * a.path_bytes);
         double *const to = f == 0 ? g.r : f < 5 ? g.c1 + (f - 1) * (FM_MAX_LEGS + 1) : g.cb + (f - 5) * (FM_MAX_LEGS + 1);
-        to[J] = get_double(w + 2 * x);
+        to[J] = t;
     }
-    if (lane <= n) {
-        const uint32_t v = w[2 * (9 * n + 3) + lane];     // ok, then the potentials
-        if (lane == 0) { g.ok = (int)v; g.n = n; } else g.ipot[lane - 1] = (int)v;
-        if (lane == 1) g.ipot[n] = (int)v;
-    }
-    if (lane < 3) {
-        const double v = get_double(w + 2 * (9 * n + lane));
-        if (lane == 0) g.R = v; else if (lane == 1) g.reff = v; else g.prod_r = v;
+    if (q < np) {
+        PathLDS &g = *reinterpret_cast<PathLDS *>(smem + (size_t)j * a.path_bytes);
+        if (k == 0) {
+            g.R = d;
+            g.n = n;
+            pidx[j] = p;
+            pval[j] = valid ? 1 : 0;
+        } else if (k == 1) {
+            g.reff = d;
+        } else if (k == 2) {
+            g.prod_r = d;
+        } else if (k == 3) {
+            g.ok = (int)v;
+        } else {
+            g.ipot[k - 4] = (int)v;
+            if (k == 4) g.ipot[n] = (int)v;
+        }
     }
 }
 // The fine grid of the paths whose rows hold cchi, one wavefront per path.
@@ -194,6 +221,9 @@ __global__ __launch_bounds__(FM_WAVE * 4) __attribute__((amdgpu_waves_per_eu(FM_
             int ei;
             load_path_group(a.src, p, g, ei, nl, lane & 15, act, false);   // single scattering: no tables
             if (act && (lane & 15) == 0) { pidx[j] = p; pval[j] = valid ? 1 : 0; }
+        } else if constexpr (SPLIT) {
+            load_records(a, blk, G, wid, lane, smem, pidx, pval);
+            wave_sync();
         } else {
             for (int j = wid; j < G; j += 4) {
                 const int slot = blk * G + j;
@@ -201,17 +231,15 @@ __global__ __launch_bounds__(FM_WAVE * 4) __attribute__((amdgpu_waves_per_eu(FM_
                 const int s0 = valid ? slot : blk * G;
                 const int p = a.order ? a.order[a.first + s0] : a.first + s0;
                 PathLDS &g = *reinterpret_cast<PathLDS *>(smem + (size_t)j * a.path_bytes);
-                if constexpr (SPLIT) {
-                    load_record(a, p, g, lane);
-                } else {
-                    int ei;
-                    load_path(a.src, p, g, ei, nl);
-                }
+                int ei;
+                load_path(a.src, p, g, ei, nl);
                 if (lane == 0) { pidx[j] = p; pval[j] = valid ? 1 : 0; }
             }
-            if constexpr (SPLIT) wave_sync();
         }
-        if constexpr (SET < FM_SET_SS) build_tables<T, SET, false, 1>(ed, smem, a.path_bytes, off_W, 0, wid, 4, G, nl, ltab);
+        // the tables' coefficients 8 rows at a time in a split launch (which keeps matrices 6% faster than row by row; the
+        // unsplit kernel, short of registers, is faster row by row)
+        if constexpr (SET < FM_SET_SS)
+            build_tables<T, SET, false, SPLIT ? 8 : 1>(ed, smem, a.path_bytes, off_W, 0, wid, 4, G, nl, ltab);
         __syncthreads();
         // ---- energies: the bands of this wavefront, each wavefront stepping from one of its bands to the next
         auto next_band = [&](int b) {
