@@ -745,13 +745,10 @@ int fm_chi_paths_overlap(const fm_edge *edges, int32_t nedge, const fm_paths *pa
     if (hipError_t e = lanes.join()) return hip_err(e, "fm_chi_paths side streams");
     if (chi_seg && nseg > 0) {
         if (!seg_ptr || !seg_paths) return set_err(FM_EINVAL, "NULL segment lists");
-        dim3 grd((grid->nk + FM_WAVE - 1) / FM_WAVE, nseg);
         if (precision == 32)
-            hipLaunchKernelGGL(k_segment_sum<float>, grd, dim3(FM_WAVE * SEG_WAVES), 0, st, nseg, grid->nk, seg_ptr, seg_paths,
-                               paths->deg, (const float *)chi_path, chi_seg);
+            launch_segment_sum(nseg, grid->nk, seg_ptr, seg_paths, paths->deg, (const float *)chi_path, chi_seg, st);
         else
-            hipLaunchKernelGGL(k_segment_sum<double>, grd, dim3(FM_WAVE * SEG_WAVES), 0, st, nseg, grid->nk, seg_ptr, seg_paths,
-                               paths->deg, (const double *)chi_path, chi_seg);
+            launch_segment_sum(nseg, grid->nk, seg_ptr, seg_paths, paths->deg, (const double *)chi_path, chi_seg, st);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return hip_err(e, "segment sum launch");
     }

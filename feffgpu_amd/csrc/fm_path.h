@@ -814,27 +814,31 @@ __device__ void fine_grid(const fm_edge &ed, const int32_t *jq, const double *fq
 }
 
 
-// chi_seg[s][k] = sum over the CSR list of segment s of deg[p] chi_path[p][k]: a workgroup per (64 k-points,
-// segment); wave w sums the list entries w, w + 8, ... in order, then the 8 partial sums are added in wave order.
-// Deterministic for a given list and grid.
+// chi_seg[s][k] = sum over the CSR list of segment s of deg[p] chi_path[p][k]: a workgroup per (KL k-points, segment);
+// part x of its 16 64 / KL sums the list entries x, x + parts, ... in order, then the parts are added in order.
+// Deterministic for a given list and grid. Bound by the latency of three dependent loads per batch of 16 entries: with
+// few workgroups of 64 k-points (fewer than SEG_NARROW) KL = 16 puts four times as many, of a quarter of the batches, on
+// the chip (KL = 64 / 16, us: 1 segment of a bcc cluster 25 / 10, 8 segments of MD frames 32 / 17; 64 segments of 1472
+// paths, which fill the chip either way, 65 / 74).
 constexpr int SEG_WAVES = 16;
-template <class T>
+template <class T, int KL>
 __global__ __launch_bounds__(FM_WAVE *SEG_WAVES) void k_segment_sum(int nseg, int nk, const int32_t *seg_ptr,
                                                                      const int32_t *seg_paths, const double *deg,
                                                                      const T *chi_path, double *chi_seg) {
-    __shared__ double part[SEG_WAVES][FM_WAVE];
+    constexpr int NP = SEG_WAVES * FM_WAVE / KL;
+    __shared__ double part[NP][KL];
     const int s = blockIdx.y;
-    const int w = threadIdx.x / FM_WAVE, lane = threadIdx.x % FM_WAVE;
-    const int k = blockIdx.x * FM_WAVE + lane;
+    const int w = threadIdx.x / KL, lane = threadIdx.x % KL;
+    const int k = blockIdx.x * KL + lane;
     double acc = 0.0;
     if (k < nk) {
         const int t0 = seg_ptr[s] + w, t1 = seg_ptr[s + 1];
         constexpr int U = 16;   // paths whose loads are in flight together; summed in list order
-        for (int tb = t0; tb < t1; tb += U * SEG_WAVES) {
+        for (int tb = t0; tb < t1; tb += U * NP) {
             int pv[U];
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                const int t = tb + u * SEG_WAVES;
+                const int t = tb + u * NP;
                 pv[u] = t < t1 ? seg_paths[t] : -1;
             }
             // unconditional loads (past the list's end they read path 0, a valid row, and are not summed), so that
@@ -855,9 +859,21 @@ __global__ __launch_bounds__(FM_WAVE *SEG_WAVES) void k_segment_sum(int nseg, in
     __syncthreads();
     if (w == 0 && k < nk) {
         double tot = 0.0;
-        for (int i = 0; i < SEG_WAVES; ++i) tot += part[i][lane];
+        for (int i = 0; i < NP; ++i) tot += part[i][lane];
         chi_seg[(size_t)s * nk + k] = tot;
     }
+}
+constexpr long SEG_NARROW = 256;
+template <class T>
+inline void launch_segment_sum(int nseg, int nk, const int32_t *seg_ptr, const int32_t *seg_paths, const double *deg,
+                               const T *chi_path, double *chi_seg, hipStream_t st) {
+    const int blocks = (nk + FM_WAVE - 1) / FM_WAVE;
+    if ((long)nseg * blocks < SEG_NARROW)
+        hipLaunchKernelGGL((k_segment_sum<T, 16>), dim3((nk + 15) / 16, nseg), dim3(FM_WAVE * SEG_WAVES), 0, st, nseg, nk,
+                           seg_ptr, seg_paths, deg, chi_path, chi_seg);
+    else
+        hipLaunchKernelGGL((k_segment_sum<T, FM_WAVE>), dim3(blocks, nseg), dim3(FM_WAVE * SEG_WAVES), 0, st, nseg, nk,
+                           seg_ptr, seg_paths, deg, chi_path, chi_seg);
 }
 
 }  // namespace fm

@@ -481,9 +481,7 @@ int fm_chi_paths_plain(const fm_edge *edges, int32_t nedge, const fm_paths *path
     }
     if (chi_seg && nseg > 0) {
         if (!seg_ptr || !seg_paths) return set_err(FM_EINVAL, "NULL segment lists");
-        dim3 grd((grid->nk + FM_WAVE - 1) / FM_WAVE, nseg);
-        hipLaunchKernelGGL(k_segment_sum<double>, grd, dim3(FM_WAVE * SEG_WAVES), 0, st, nseg, grid->nk, seg_ptr, seg_paths,
-                           paths->deg, (const double *)chi_path, chi_seg);
+        launch_segment_sum(nseg, grid->nk, seg_ptr, seg_paths, paths->deg, (const double *)chi_path, chi_seg, st);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return hip_err(e, "segment sum launch");
     }
