@@ -164,9 +164,9 @@ enum { FM_BUCKET_K_MS = 0, FM_BUCKET_LM_MS = 1, FM_BUCKET_SS = 2 };
  * workgroups, -1 as many as the device's CUs hold at once, that loop over the groups. tickets (device, two uint32,
  * zero before first use; used only with grid != 0): the groups are then taken from this counter one at a time, and
  * the launch's last workgroup puts the pair back to zero, so it can serve every later launch on the same stream (not
- * two launches that overlap in time); NULL: workgroup i takes groups i, i + grid, ... The multiple-scattering
- * adjoint of 3-6 legs (and single scattering) applies the policy to its sweep; its per-path tail runs one wavefront
- * per path.
+ * two launches that overlap in time); NULL: workgroup i takes groups i, i + grid, ... The forward of a long
+ * list and the adjoint of single scattering apply the policy to their kernel over the energies, the adjoint of 3-6
+ * legs to the one that rebuilds the scattering matrices where none are kept; their other kernels have a fixed split.
  * keep (device, keep_bytes >= fm_keep_bytes(precision, edge, nleg, paths of the bucket)), for buckets of multiple
  * scattering of 3-6 legs (ignored by the others): fm_chi_paths writes the scattering matrices of every path's
  * scatterers into it ([path][row][energy] complex, paths in bucket order; the rows of a path are the independent
