@@ -22,8 +22,9 @@
 // chain's matrices, one wavefront per SIMD), so two wavefronts share a SIMD; its units are many and small, which
 // balances the very uneven numbers of partial waves per energy (5 to 29 on a K edge); and its sums need no per-energy
 // slots in memory. K costs one write and one read of as many bytes as the kept matrices. Against the one-kernel sweep
-// that this replaces (MI355X, FP32, all paths of the bucket, us): K edge 3 legs 4608 paths, 2430 -> 1560 (chain 506,
-// stream 680, pbc 353, setup and geometry 57); a NiO box of 2-4 legs, whole step, 21.6 -> 17.0 ms; FP64 2.30 -> 1.63 ms.
+// that this replaces (MI355X, FP32, us): 94 304 K-edge paths of 3 legs, 3570 -> 2470 (chain 750 at 3.9 TB/s, stream 1046
+// with the vector pipes 88 % busy, pbc 537, setup 71, geometry 66); a NiO box of 2-4 legs, whole step, 21.6 -> 17.0 ms;
+// the same in FP64 on a smaller box 2.30 -> 1.63 ms.
 //
 // The single-precision sums of this file keep their roundings to the last bit from one layout of the work to the next:
 // where the compiler's choice of the product that a fused multiply-add takes depends on what it shares with its
