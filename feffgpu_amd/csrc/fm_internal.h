@@ -52,7 +52,7 @@ struct Lanes {
     int n = 1;
     hipError_t err = hipSuccess;
     Lanes(fm_overlap *o, hipStream_t st, int want);
-    ~Lanes() { join(); }
+    ~Lanes() { (void)join(); }
     Lanes(const Lanes &) = delete;
     hipStream_t at(int lane) const { return lane == 0 || lane >= n ? st : o->side[lane - 1]; }
     hipError_t join();

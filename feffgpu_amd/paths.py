@@ -236,8 +236,12 @@ class PathPlan:
                 beside = int(N.lib().fm_backward_overlap_bytes(self.precision, self.edge_array, nbk, self._h_off,
                                                                self._h_edge, self._h_nlm, int(self.keep_amplitudes)))
         big = int(np.diff(self.buckets.offset).max()) if Pn else 0
-        self.workspace = N.backward_workspace(self.precision, nmax, big, dev, max(T.E for T in self.tables),
-                                              at_least=beside if beside <= OVERLAP_BYTES else 0) if Pn else None
+        maxe = max(T.E for T in self.tables)
+        try:
+            self.workspace = N.backward_workspace(self.precision, nmax, big, dev, maxe,
+                                                  at_least=beside if beside <= OVERLAP_BYTES else 0) if Pn else None
+        except torch.cuda.OutOfMemoryError:     # the adjoint's buckets one after the other in the smaller one
+            self.workspace = N.backward_workspace(self.precision, nmax, big, dev, maxe)
         # per-bucket launch policies of the forward (0) and adjoint (1) calls: defaults until set_launch / tune;
         # every bucket and kernel has its own zeroed counter pair for persistent launches that take groups in turn
         nb = max(1, len(self.buckets.kind))

@@ -115,3 +115,18 @@ def test_two_threads_and_returned_sets():
     [t.join() for t in th]
     for s in (1, 2):
         assert all(torch.equal(a, b) for a, b in zip(got[s], want[s]))
+
+
+def test_no_room_for_the_lanes(monkeypatch):
+    """A device without room for a region per lane gets the smaller workspace and the same results."""
+    from feffgpu_amd import _native as N
+    plan, p, g = _plan(5)
+    want, real = _run(plan, p, g), N.backward_workspace
+
+    def full(*a, at_least=0, **k):
+        if at_least:
+            raise torch.cuda.OutOfMemoryError("no room")
+        return real(*a, **k)
+    monkeypatch.setattr(N, "backward_workspace", full)
+    plan, p, g = _plan(5)
+    assert all(torch.equal(a, b) for a, b in zip(_run(plan, p, g), want))
