@@ -231,6 +231,7 @@ class MultipleScattering:
         self.row_of[self.abs_atoms] = torch.arange(C * A, device=self.device)
         self.counts = {nleg: int(v["atoms"].shape[0]) for nleg, v in self.lists.items()}
         self._plans = {}
+        self.full._plans = {}        # the plans are built and held there; those of the previous lists go
         return self.counts
 
     def set_cell(self, box):
