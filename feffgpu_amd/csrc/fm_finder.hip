@@ -735,7 +735,7 @@ int fm_find_filter(int64_t npath, const float *dtot, const float *xport, const i
 int fm_find_ref(int32_t nabs, int64_t npath, const int32_t *slot, const float *len, const float *xport, const float *deg,
                 const int32_t *ncand, int32_t merged, float *ref, void *stream) {
     if (nabs <= 0) return FM_OK;
-    if (!ref || npath < 0 || (npath > 0 && (!slot || !len || !xport)) || (merged && (!deg || !ncand)))
+    if (!ref || npath < 0 || (npath > 0 && (!slot || !len || !xport || (merged && !deg))) || (merged && !ncand))
         return fm_set_err(FM_EINVAL, "fm_find_ref: bad arguments");
     hipLaunchKernelGGL(k_find_ref, dim3(nabs), dim3(64), 0, (hipStream_t)stream, nabs, npath, slot, len, xport, deg, ncand,
                        merged, ref);
