@@ -178,6 +178,7 @@ def lib():
         L.fm_pair_chi_workspace_bytes.argtypes = [_i32, _i32, _i32]
         L.fm_pair_chi.argtypes = [_i32, _P(_vp), _P(_i32), _i32, _i32, _i32, _vp, _i32, ctypes.c_double, _vp, _vp, _sz,
                                   _vp]
+        L.fm_pair_chi_held.argtypes = L.fm_pair_chi.argtypes[:10] + [_vp] + L.fm_pair_chi.argtypes[10:]
         L.fm_pair_chi_grad.argtypes = [_i32, _P(_vp), _P(_i32), _i32, _i32, _i32, _vp, ctypes.c_double, _vp, _vp]
         L.fm_set_lds_budget.restype = _i32
         L.fm_set_lds_budget.argtypes = [_i32, _i32]

@@ -373,24 +373,34 @@ __global__ __launch_bounds__(FM_WAVE *PG_WAVES) void k_pair_grad(int natom, cons
 // chi[k] = sum_i hist[i] table[i][k] / div over the rows i of one potential's table: a workgroup sums TS_ROWS rows of
 // 64 points (its wavefronts interleaved over the rows, their sums added in order) into part[chunk][k]; k_table_total
 // adds the chunks of every potential in order. TT: the tables' type, HT: int64 fixed point (2^-32) or double.
-// Reading the table once is the bound (5.7 MB per potential, 1.2 us at 4.7 TB/s); at 4.6 us it is mostly launch
+// Reading the table once is the bound (5.7 MB per potential, 1.2 us at 4.7 TB/s); at 3.8 us it is mostly launch
 // latency (the stacked FP64 copy of the tables, its transpose and library products it replaces took about 100 us).
+// held: a copy of the table made on the way, or NULL (6.0 us with it; a copy of two tables by launches of their own added
+// 18 us to a call).
 constexpr int TS_ROWS = 128, TS_WAVES = 8;
 template <class HT> __device__ __forceinline__ double hist_value(HT h) { return (double)h; }
 template <> __device__ __forceinline__ double hist_value<long long>(long long h) { return (double)h * (1.0 / PH_ONE); }
 template <class TT, class HT>
 __global__ __launch_bounds__(FM_WAVE *TS_WAVES) void k_table_sum(int nr, int nk, const TT *table, const HT *hist,
-                                                                 double *part) {
+                                                                 double *part, TT *held) {
     __shared__ double sm[TS_WAVES][FM_WAVE];
     const int w = threadIdx.x / FM_WAVE, lane = threadIdx.x % FM_WAVE;
     const int k = blockIdx.x * FM_WAVE + lane, i0 = blockIdx.y * TS_ROWS;
+    TT x[TS_ROWS / TS_WAVES];
     double acc = 0.0;
 #pragma unroll
     for (int u = 0; u < TS_ROWS / TS_WAVES; ++u) {
         const int i = i0 + u * TS_WAVES + w, ic = i < nr ? i : nr - 1;
         const double h = hist_value(hist[ic]);
-        const double v = (double)table[(size_t)ic * nk + (k < nk ? k : nk - 1)];
-        acc += i < nr ? h * v : 0.0;
+        x[u] = table[(size_t)ic * nk + (k < nk ? k : nk - 1)];
+        acc += i < nr ? h * (double)x[u] : 0.0;
+    }
+    if (held && k < nk) {
+#pragma unroll
+        for (int u = 0; u < TS_ROWS / TS_WAVES; ++u) {
+            const int i = i0 + u * TS_WAVES + w;
+            if (i < nr) held[(size_t)i * nk + k] = x[u];
+        }
     }
     sm[w][lane] = acc;
     __syncthreads();
@@ -517,6 +527,13 @@ size_t fm_pair_chi_workspace_bytes(int32_t npot, int32_t nr, int32_t nk) {
 int fm_pair_chi(int32_t npot, const void *const *tables, const int32_t *rows, int32_t precision, int32_t nr, int32_t nk,
                 const void *hist, int32_t fixed_point, double div, double *chi, void *workspace, size_t workspace_bytes,
                 void *stream) {
+    return fm_pair_chi_held(npot, tables, rows, precision, nr, nk, hist, fixed_point, div, chi, nullptr, workspace,
+                            workspace_bytes, stream);
+}
+
+int fm_pair_chi_held(int32_t npot, const void *const *tables, const int32_t *rows, int32_t precision, int32_t nr,
+                     int32_t nk, const void *hist, int32_t fixed_point, double div, double *chi, void *held,
+                     void *workspace, size_t workspace_bytes, void *stream) {
     if (npot < 1 || nr < 1 || nk < 1) return fm_set_err(FM_EINVAL, "fm_pair_chi: bad sizes");
     if (precision != 32 && precision != 64) return fm_set_err(FM_EINVAL, "precision must be 32 or 64");
     if (!tables || !rows || !hist || !chi || !workspace) return fm_set_err(FM_EINVAL, "fm_pair_chi: NULL buffer");
@@ -529,18 +546,25 @@ int fm_pair_chi(int32_t npot, const void *const *tables, const int32_t *rows, in
     for (int p = 0; p < npot; ++p) {
         if (!tables[p] || rows[p] < 0) return fm_set_err(FM_EINVAL, "fm_pair_chi: NULL table or negative row");
         double *const out = part + (size_t)p * chunks * nk;
+        const size_t at = (size_t)p * nr * nk;
+        float *const h32 = held ? (float *)held + at : nullptr;
+        double *const h64 = held ? (double *)held + at : nullptr;
         if (fixed_point) {
             const long long *h = (const long long *)hist + (size_t)rows[p] * nr;
             if (precision == 32)
-                hipLaunchKernelGGL((k_table_sum<float, long long>), grd, blk, 0, st, nr, nk, (const float *)tables[p], h, out);
+                hipLaunchKernelGGL((k_table_sum<float, long long>), grd, blk, 0, st, nr, nk, (const float *)tables[p], h,
+                                   out, h32);
             else
-                hipLaunchKernelGGL((k_table_sum<double, long long>), grd, blk, 0, st, nr, nk, (const double *)tables[p], h, out);
+                hipLaunchKernelGGL((k_table_sum<double, long long>), grd, blk, 0, st, nr, nk, (const double *)tables[p],
+                                   h, out, h64);
         } else {
             const double *h = (const double *)hist + (size_t)rows[p] * nr;
             if (precision == 32)
-                hipLaunchKernelGGL((k_table_sum<float, double>), grd, blk, 0, st, nr, nk, (const float *)tables[p], h, out);
+                hipLaunchKernelGGL((k_table_sum<float, double>), grd, blk, 0, st, nr, nk, (const float *)tables[p], h,
+                                   out, h32);
             else
-                hipLaunchKernelGGL((k_table_sum<double, double>), grd, blk, 0, st, nr, nk, (const double *)tables[p], h, out);
+                hipLaunchKernelGGL((k_table_sum<double, double>), grd, blk, 0, st, nr, nk, (const double *)tables[p],
+                                   h, out, h64);
         }
     }
     hipLaunchKernelGGL(k_table_total, dim3((unsigned)((nk + FM_WAVE * 4 - 1) / (FM_WAVE * 4))), dim3(FM_WAVE * 4), 0, st,

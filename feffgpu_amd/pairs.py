@@ -197,23 +197,29 @@ class _SingleScattering(torch.autograd.Function):
         ptrs, rows, prec = _table_args(T, pots, pt.nr)
         nk = T[0].shape[1]
         L = N.lib()
+        # the gradient is that of the tables as they are now: a copy of them where they are the caller's own tensors
+        held = None
+        if ctx.needs_input_grad[0] and any(t is pt.tables[p] for p, t in zip(pots, T)):
+            held = torch.empty(len(T), pt.nr, nk, dtype=tt, device=pos.device)
         ws = torch.empty(int(L.fm_pair_chi_workspace_bytes(len(T), pt.nr, nk)), dtype=torch.uint8, device=pos.device)
         chi = torch.empty(nk, dtype=torch.float64, device=pos.device)
-        N.check(L.fm_pair_chi(len(T), ptrs, rows, prec, pt.nr, nk, (hist if h is None else h).data_ptr(),
-                              1 if h is None else 0, float(C * n), chi.data_ptr(), ws.data_ptr(), ws.numel(),
-                              N.stream_of(pos.device)), "fm_pair_chi")
-        ctx.save_for_backward(P, ip, *T)
-        ctx.pt, ctx.pots, ctx.shape, ctx.dtype = pt, pots, (C, n), pos.dtype
+        N.check(L.fm_pair_chi_held(len(T), ptrs, rows, prec, pt.nr, nk, (hist if h is None else h).data_ptr(),
+                                   1 if h is None else 0, float(C * n), chi.data_ptr(), N.ptr(held), ws.data_ptr(),
+                                   ws.numel(), N.stream_of(pos.device)), "fm_pair_chi")
+        ctx.save_for_backward(P, ip, *(T if held is None else [held]))
+        ctx.pt, ctx.rows, ctx.tables, ctx.shape, ctx.dtype = pt, rows, (len(T), prec, nk), (C, n), pos.dtype
         return chi.to(pos.dtype)
 
     @staticmethod
     def backward(ctx, gchi):
         P, ip, *T = ctx.saved_tensors
-        pt, (C, n) = ctx.pt, ctx.shape
+        pt, (C, n), (nt, prec, nk) = ctx.pt, ctx.shape, ctx.tables
         gbin = torch.zeros(pt.npot, pt.nr, dtype=torch.float64, device=P.device)
         gk = gchi.to(torch.float64).contiguous()
-        ptrs, rows, prec = _table_args(T, ctx.pots, pt.nr)
-        N.check(N.lib().fm_pair_chi_grad(len(T), ptrs, rows, prec, pt.nr, T[0].shape[1], gk.data_ptr(), float(C * n),
+        step = pt.nr * nk * prec // 8
+        ptrs = (ctypes.c_void_p * nt)(*([t.data_ptr() for t in T] if T[0].dim() == 2 else
+                                        [T[0].data_ptr() + i * step for i in range(nt)]))
+        N.check(N.lib().fm_pair_chi_grad(nt, ptrs, ctx.rows, prec, pt.nr, nk, gk.data_ptr(), float(C * n),
                                          gbin.data_ptr(), N.stream_of(P.device)), "fm_pair_chi_grad")
         grad = torch.empty(C, n, 3, dtype=torch.float64, device=P.device)
         g = pt._grid()

@@ -299,6 +299,12 @@ int fm_pair_chi(int32_t npot, const void *const *tables, const int32_t *rows, in
                 const void *hist, int32_t fixed_point, double div, double *chi, void *workspace, size_t workspace_bytes,
                 void *stream);
 
+/* The same with a copy of the tables in held (device, [npot][nr][nk] of their type; NULL: none), for an adjoint of the
+ * tables as they were at this call. */
+int fm_pair_chi_held(int32_t npot, const void *const *tables, const int32_t *rows, int32_t precision, int32_t nr,
+                     int32_t nk, const void *hist, int32_t fixed_point, double div, double *chi, void *held,
+                     void *workspace, size_t workspace_bytes, void *stream);
+
 /* Its adjoint in the bins: gbin[rows[p]][i] = sum_k tables[p][i][k] gchi[k] / div for the npot rows (others untouched). */
 int fm_pair_chi_grad(int32_t npot, const void *const *tables, const int32_t *rows, int32_t precision, int32_t nr,
                      int32_t nk, const double *gchi, double div, double *gbin, void *stream);
