@@ -368,6 +368,7 @@ __global__ void k_scan_add(int64_t *out, int64_t n, const int64_t *sums) {
 // the energies. The criterion is a chain of divisions and table reads per energy, and a list has few paths for the chip:
 // one thread per path was bound by that latency (7 000 to 30 000 paths, 75 energies: 42 to 63 us, here 10).
 constexpr int IM_LANES = 8;
+constexpr int64_t IM_PATHS = (int64_t)1 << 28;     // of one launch, whose threads must stay below 2^32
 template <int NLEG>
 __global__ __launch_bounds__(256) void k_find_importance(fm_find_tables t, int64_t npath, const float *coords,
                                                          const int64_t *ipots, float *xport, float *rtot_out) {
@@ -682,8 +683,11 @@ int fm_find_importance(const fm_find_tables *t, int64_t npath, int32_t nleg, con
         return fm_set_err(FM_EINVAL, "fm_find_importance: NULL buffer");
     if (nleg < 2 || nleg > FM_MAX_LEGS) return fm_set_err(FM_EINVAL, "fm_find_importance: nleg out of range 2..9");
     const auto run = [&](auto k) {
-        hipLaunchKernelGGL(k, dim3(blocks_of(npath * IM_LANES, 256)), dim3(256), 0, (hipStream_t)stream, *t, npath, coords,
-                           ipots, xport, rtot);
+        for (int64_t p = 0; p < npath; p += IM_PATHS) {
+            const int64_t n = npath - p < IM_PATHS ? npath - p : IM_PATHS;
+            hipLaunchKernelGGL(k, dim3(blocks_of(n * IM_LANES, 256)), dim3(256), 0, (hipStream_t)stream, *t, n,
+                               coords + p * nleg * 3, ipots + p * nleg, xport + p, rtot ? rtot + p : nullptr);
+        }
     };
     switch (nleg) {
         case 2: run(k_find_importance<2>); break;
