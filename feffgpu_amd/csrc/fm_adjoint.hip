@@ -1022,6 +1022,7 @@ template <class T, int SET, int NL> hipError_t launch_nl(const MsAdjoint &m, MAr
     if (r < group + 2048) return hipErrorOutOfMemory;
     long chunk = (long)((r - 2048) / group) * KG;
     if (chunk > m.npath) chunk = m.npath;
+    if (chunk > (1 << 23)) chunk = 1 << 23;     // k_chain: at most 4 wavefronts per path, fewer than 2^32 threads
     const size_t np = (size_t)((chunk + KG - 1) / KG) * KG;
     unsigned char *w = m.work;
     auto take = [&](size_t bytes) {

@@ -82,6 +82,7 @@ int hip_err(hipError_t e, const char *where) {
 // potentials; after the bands the row holds cchi (2 E of T), reff (A) and ok. 32-bit words: rows need not be 8-byte
 // aligned.
 constexpr int SPLIT_MIN = 1280;
+constexpr int SPLIT_PATHS = 1 << 25;     // of one launch of k_rows or k_fine, whose threads must stay below 2^32
 __host__ __device__ constexpr int rec_words(int n) { return 2 * (9 * n + 3) + n + 1; }
 __device__ __forceinline__ void put_double(uint32_t *w, double v) { __builtin_memcpy(w, &v, 8); }
 __device__ __forceinline__ double get_double(const uint32_t *w) {
@@ -500,12 +501,24 @@ template <class T, int SET, bool SPLIT> hipError_t launch_main(KArgs &a, const f
     if (e != hipSuccess) return e;
     if (blocks == 0) return hipSuccess;
     a.tickets = pol.grid != 0 ? pol.tickets : nullptr;
+    const auto pieces = [&](auto run) {
+        for (long f = 0; f < a.npath_bucket; f += SPLIT_PATHS) {
+            KArgs b = a;
+            b.first = a.first + (int)f;
+            b.npath_bucket = a.npath_bucket - f < SPLIT_PATHS ? (int)(a.npath_bucket - f) : SPLIT_PATHS;
+            run(b);
+        }
+    };
     if (SPLIT && SET < FM_SET_SS)
-        hipLaunchKernelGGL(k_rows, dim3((unsigned)((a.npath_bucket + 15) / 16)), dim3(256), 0, st, a);
+        pieces([&](const KArgs &b) {
+            hipLaunchKernelGGL(k_rows, dim3((unsigned)((b.npath_bucket + 15) / 16)), dim3(256), 0, st, b);
+        });
     hipLaunchKernelGGL((k_forward<T, SET, SPLIT>), dim3((unsigned)blocks), dim3(FM_WAVE * 4), shm, st, a);
     if (SPLIT && a.src.mode == 1) {
         const size_t wb = align16(sizeof(T) * (size_t)ed.E) + align16(sizeof(double) * (size_t)ed.E);
-        hipLaunchKernelGGL(k_fine<T>, dim3((unsigned)((a.npath_bucket + 3) / 4)), dim3(FM_WAVE * 4), 4 * wb, st, a, wb);
+        pieces([&](const KArgs &b) {
+            hipLaunchKernelGGL(k_fine<T>, dim3((unsigned)((b.npath_bucket + 3) / 4)), dim3(FM_WAVE * 4), 4 * wb, st, b, wb);
+        });
     }
     return hipGetLastError();
 }

@@ -115,9 +115,11 @@ inline int choose_gpaths(const fm_edge &e, size_t path_bytes, size_t budget, int
 
 // Workgroups of a launch over `groups` path groups: one per group (grid 0), or a persistent grid of `grid`
 // workgroups (-1: as many as the device's CUs hold at once with this kernel's registers and `shm` bytes of LDS),
-// never more than the groups. The kernel's dynamic LDS limit must already allow `shm`.
+// never more than the groups or than 2^32 threads take (the workgroups loop over the groups). The kernel's dynamic LDS
+// limit must already allow `shm`.
 inline hipError_t launch_grid(const void *fn, size_t shm, long groups, int grid, long *out) {
-    *out = groups;
+    constexpr long MAX_BLOCKS = ((long)1 << 32) / (FM_WAVE * 4) - 1;
+    *out = groups < MAX_BLOCKS ? groups : MAX_BLOCKS;
     if (grid == 0 || groups == 0) return hipSuccess;
     long g = grid;
     if (grid < 0) {
@@ -128,7 +130,7 @@ inline hipError_t launch_grid(const void *fn, size_t shm, long groups, int grid,
         if (e != hipSuccess) return e;
         g = (long)(cus > 0 ? cus : 1) * (per > 0 ? per : 1);
     }
-    if (g < groups) *out = g;
+    if (g < *out) *out = g;
     return hipSuccess;
 }
 
