@@ -200,20 +200,33 @@ def ptr(t) -> int | None:
     return None if t is None else t.data_ptr()
 
 
-def backward_workspace(precision: int, nlegmax: int, npath: int, device, E: int, max_slots: int = 4096,
-                       max_region_bytes: int = 2 << 30, at_least: int = 0):
-    """A device buffer for the adjoints: paths of 7-9 legs, band slots for the workgroups in flight (a workgroup takes
-    one per band of its plan, at most 16), at most max_slots and no more than npath workgroups need; paths of 2-6 legs,
-    for each of up to npath paths of a launch the chain's matrices, the scattering matrices and cchi of an adjoint whose
-    forward kept none, and a record, at most max_region_bytes (larger buckets run in chunks); at_least bytes."""
+def backward_bytes(precision: int, nlegmax: int, npath: int, E: int, max_slots: int = 4096,
+                   max_region_bytes: int = 1 << 30) -> int:
+    """Bytes of a workspace for the adjoints: paths of 7-9 legs, band slots for the workgroups in flight (a workgroup
+    takes one per band of its plan, at most 16), at most max_slots and no more than npath workgroups need; paths of 2-6
+    legs, for each of up to npath paths of a launch the chain's matrices, the scattering matrices and cchi of an adjoint
+    whose forward kept none, and a record, at most max_region_bytes (larger buckets run in chunks)."""
     slots = max(16, min(int(max_slots), 16 * max(int(npath), 1))) if nlegmax > 6 else 16
     nbytes = lib().fm_backward_workspace_bytes(int(precision), int(nlegmax), slots)
     n, ec = min(int(nlegmax), 6), 8 if precision == 32 else 16
     per = 9 * int(E) * ec
     if n > 2:
         per = max(per, (40 * (n - 1) + n + 4) * (int(E) + 3) * ec + 8 * (10 * n + 5) + ec // 2 * (4 * n + 160))
-    nbytes = max(nbytes, min((int(npath) + 32) * per, int(max_region_bytes)))
-    return torch.empty(max(nbytes, int(at_least), 1), dtype=torch.uint8, device=device)
+    return max(nbytes, min((int(npath) + 32) * per, int(max_region_bytes)), 1)
+
+
+def backward_workspace(precision: int, nlegmax: int, npath: int, device, E: int, max_slots: int = 4096,
+                       max_region_bytes: int = 1 << 30, at_least: int = 0):
+    """A device buffer of backward_bytes, of what the adjoints need at least where the device has no room for that; or
+    of at_least bytes, if that is more."""
+    nbytes = backward_bytes(precision, nlegmax, npath, E, max_slots, max_region_bytes)
+    try:
+        return torch.empty(max(nbytes, int(at_least)), dtype=torch.uint8, device=device)
+    except torch.cuda.OutOfMemoryError:
+        if at_least > nbytes:
+            raise
+        least = int(lib().fm_backward_workspace_bytes(int(precision), int(nlegmax), 16))
+        return torch.empty(max(least, 1), dtype=torch.uint8, device=device)
 
 
 def stream_of(device) -> int:

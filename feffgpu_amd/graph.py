@@ -2,9 +2,10 @@
 its adjoint, replayed on static buffers.
 
 Every launch of a step is stream-ordered and allocation-free once the plan's buffers exist (fm_chi_paths,
-fm_chi_paths_backward, torch's elementwise kernels; no memset nodes, no host synchronisation), so the sequence
-captures as one graph: bucket kernels, segment sum, the loss gradient, adjoint kernels, per-atom gradient sum. A
-replay re-reads `pos` (and `gseg`) from the same device addresses; copy new values into them before replaying.
+fm_chi_paths_backward, torch's elementwise kernels; no memset nodes, no host synchronisation; what a call's tensors
+take, a long list's adjoint workspace among them, is the graph's own memory), so the sequence captures as one graph:
+bucket kernels, segment sum, the loss gradient, adjoint kernels, per-atom gradient sum. A replay re-reads `pos` (and
+`gseg`) from the same device addresses; copy new values into them before replaying.
 
     step = CapturedStep(plan, natom, loss_grad=lambda seg: 2 * w * (seg - target))
     step.pos.copy_(pos)            # or step(pos)

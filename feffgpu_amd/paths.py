@@ -27,7 +27,9 @@ from . import _native as N
 from .pad import load_phase
 from .tables import edge_tables, energies_needed, interpolation, spline_matrix
 
-OVERLAP_BYTES = 8 << 30    # the largest adjoint workspace for buckets that run next to each other
+HELD_BYTES = 1 << 30       # the largest adjoint workspace that a plan holds
+OVERLAP_BYTES = 8 << 30    # the largest that one call takes for buckets that run next to each other
+REGION_BYTES = 2 << 30     # ... and for one bucket after the other
 
 
 def _cell_struct(cell):
@@ -237,11 +239,9 @@ class PathPlan:
                                                                self._h_edge, self._h_nlm, int(self.keep_amplitudes)))
         big = int(np.diff(self.buckets.offset).max()) if Pn else 0
         maxe = max(T.E for T in self.tables)
-        try:
-            self.workspace = N.backward_workspace(self.precision, nmax, big, dev, maxe,
-                                                  at_least=beside if beside <= OVERLAP_BYTES else 0) if Pn else None
-        except torch.cuda.OutOfMemoryError:     # the adjoint's buckets one after the other in the smaller one
-            self.workspace = N.backward_workspace(self.precision, nmax, big, dev, maxe)
+        self.workspace, self._call_bytes = None, 0
+        if Pn:
+            self._hold_workspace(big, maxe, beside)
         # per-bucket launch policies of the forward (0) and adjoint (1) calls: defaults until set_launch / tune;
         # every bucket and kernel has its own zeroed counter pair for persistent launches that take groups in turn
         nb = max(1, len(self.buckets.kind))
@@ -252,6 +252,33 @@ class PathPlan:
         # counts those calls, so that an adjoint can tell whether the matrices are still those of its forward
         self._keep = None
         self.kept_generation = 0
+
+    def _hold_workspace(self, npath, E, beside):
+        """The adjoint's workspace: held up to HELD_BYTES. A call that runs without chunks, or its buckets next to each
+        other (`beside` bytes), in more than that takes it from torch's allocator and gives it back (_call_bytes), so
+        that a plan of a long list does not hold gigabytes that its caller may want next. Not where that is more than a
+        quarter of what is free: a captured call's stays with its graph."""
+        args = (self.precision, self.nmax, npath)
+        try:
+            self.workspace = N.backward_workspace(*args, self.device, E, max_region_bytes=HELD_BYTES,
+                                                  at_least=beside if beside <= HELD_BYTES else 0)
+        except torch.cuda.OutOfMemoryError:     # the adjoint's buckets one after the other in the smaller one
+            self.workspace = N.backward_workspace(*args, self.device, E, max_region_bytes=HELD_BYTES)
+            return
+        want = max(N.backward_bytes(*args, E, max_region_bytes=REGION_BYTES), beside if beside <= OVERLAP_BYTES else 0)
+        if want > self.workspace.numel():
+            free = (torch.cuda.mem_get_info(self.device)[0] + torch.cuda.memory_reserved(self.device)
+                    - torch.cuda.memory_allocated(self.device))
+            self._call_bytes = want if want <= free // 4 else 0
+
+    def _call_workspace(self):
+        """The workspace of one adjoint call on the current stream."""
+        if self._call_bytes:
+            try:
+                return torch.empty(self._call_bytes, dtype=torch.uint8, device=self.device)
+            except torch.cuda.OutOfMemoryError:
+                pass
+        return self.workspace
 
     def set_launch(self, kernel, bucket, gpaths=0, grid=0, queue=False):
         """The launch policy of one bucket for the forward (kernel 0) or adjoint (kernel 1) calls: gpaths paths per
@@ -371,11 +398,12 @@ class PathPlan:
         if gp is not None and tuple(gp.shape) != (self.npath, self.nk):
             raise ValueError("gpath must be (P, NK)")
         ps = self._paths_struct(pos64)
+        ws = self._call_workspace()
         N.check(N.lib().fm_chi_paths_backward_overlap(
             self.edge_array, len(self.edges), ps, self.grid, self.precision, self.iorder, self.order_t.data_ptr(),
             len(self.buckets.kind), self._h_off, self._h_kind, self._h_edge, self._h_nlm, self.segment_t.data_ptr(),
             N.ptr(gs), N.ptr(gp), self.natom_ref, self.atom_ptr_t.data_ptr(), self.atom_refs_t.data_ptr(),
-            self.gcoord.data_ptr(), grad.data_ptr(), self.workspace.data_ptr(), self.workspace.numel(),
+            self.gcoord.data_ptr(), grad.data_ptr(), ws.data_ptr(), ws.numel(),
             self._policy(1, keep=kept and self._keep is not None), self._overlap, N.stream_of(self.device)),
             "fm_chi_paths_backward")
         return grad
@@ -439,10 +467,11 @@ class PathPlan:
         edge = (N._i32 * 1)(int(self.buckets.edge[b]))
         nlm = (N._i32 * 1)(int(self.buckets.nleg[b]))
         ps = self._paths_struct(pos64)
+        ws = self._call_workspace()
         N.check(N.lib().fm_chi_paths_backward(self.edge_array, len(self.edges), ps, self.grid, self.precision,
                                               self.iorder, self.order_t.data_ptr(), 1, off, kind, edge, nlm,
                                               self.segment_t.data_ptr(), gs.data_ptr(), None, 0, None, None,
-                                              self.gcoord.data_ptr(), None, self.workspace.data_ptr(), self.workspace.numel(),
+                                              self.gcoord.data_ptr(), None, ws.data_ptr(), ws.numel(),
                                               self._policy(1, b, kept and self._keep is not None),
                                               N.stream_of(self.device)), "fm_chi_paths_backward")
         return self.gcoord
