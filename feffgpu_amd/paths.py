@@ -77,6 +77,10 @@ def bucket_paths(nleg: np.ndarray, edge: np.ndarray, ilinit: list) -> Buckets:
                    np.array(nlm, np.int32))
 
 
+class _Owner:
+    pass
+
+
 class PathPlan:
     """A path list resident on the GPU, ready for repeated evaluation at new positions.
 
@@ -234,7 +238,9 @@ class PathPlan:
             with torch.cuda.device(dev):
                 self._overlap = N.lib().fm_overlap_acquire()
             if self._overlap:
-                weakref.finalize(self, N.lib().fm_overlap_release, self._overlap).atexit = False
+                # given back when the last plan that has it is gone: a shallow copy shares it as it shares the buffers
+                self._overlap_owner = _Owner()
+                weakref.finalize(self._overlap_owner, N.lib().fm_overlap_release, self._overlap).atexit = False
                 beside = int(N.lib().fm_backward_overlap_bytes(self.precision, self.edge_array, nbk, self._h_off,
                                                                self._h_edge, self._h_nlm, int(self.keep_amplitudes)))
         big = int(np.diff(self.buckets.offset).max()) if Pn else 0
