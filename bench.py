@@ -489,12 +489,14 @@ def main():
     nl = int(plan32.buckets.nleg[bdom])
     kset = int(plan32.buckets.kind[bdom]) if nl > 2 else 3 + plan32.tables[int(plan32.buckets.edge[bdom])].ilinit - 1
     summary = f"k_adjoint_{args.workload}_batch" if args.workload == "md" else f"k_adjoint_{args.workload}"
-    adj = f"k_chain<float,{kset},{nl}> + k_stream<float,{kset},{nl}>" if 3 <= nl <= 6 else f"k_adjoint<float,{kset},{nl}>"
+    adj = (f"k_setup, k_chain, k_pbc, k_stream, k_geometry <float,{kset},{nl}>" if 3 <= nl <= 6
+           else f"k_adjoint<float,{kset},{nl}>")
     traffic = measured_traffic(summary, adj)
     roof = dict(bound="valu", achieved=ach_b, peak=peak, unit="TFLOP/s", frac=ach_b / peak, traffic=traffic,
                 traffic_source=None if traffic is None else
                 f"profiles/{summary}.md (rocprofv3 FETCH_SIZE / WRITE_SIZE passes of the adjoint's kernels, copy-calibrated)",
-                kernel=f"{adj} and the launch's per-path kernels ({what})", launch_ms=t_bwd,
+                kernel=f"{adj} ({what})" if 3 <= nl <= 6 else f"{adj} and the launch's per-path kernels ({what})",
+                launch_ms=t_bwd,
                 flops_per_launch=2 * b_work[bdom], note=note)
     roof_fwd = dict(achieved=ach_f, peak=peak, unit="TFLOP/s", frac=ach_f / peak,
                     kernel=f"k_forward<float,{kset}> ({what})", launch_ms=t_fwd,
