@@ -5,7 +5,8 @@
 // The histogram is accumulated in 64-bit fixed point (units of 2^-32 of a pair): integer atomics are associative, so
 // the result does not depend on the order the pairs arrive in, and each pair adds exactly 2^32 over its two bins. A
 // bin holds up to 2^31 pairs before the signed 64-bit value overflows (the host splits larger calls). The
-// adjoint needs no atomics: one thread per atom sums its pairs, as absorber and as neighbor, in index order.
+// adjoint needs no atomics: a wavefront sums an atom's pairs, as absorber and as neighbor, over its lanes and adds the
+// lanes in a fixed order.
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <stdio.h>
@@ -176,9 +177,10 @@ __device__ __forceinline__ int lanes_below(unsigned long long m) {
 // are cleared and added to hist once per CU however many tiles there are. With every atom an absorber (absorbers
 // NULL) only pairs a < j are evaluated and added for both orders: the distance is the same to the bit (differences,
 // rint and squares are symmetric), so the integer sums are those of the ordered pairs.
-// Bound by VALU issue of the float test and the latency of a batch's gathers. 64 frames x 2000 atoms (2.56e8 ordered
-// pairs, 14.7 % within): 0.67 ms; one box of 4000 atoms: 0.041 ms (exact FP64 of every ordered pair, 64 absorbers per
-// workgroup: 2.00 ms, 0.377 ms).
+// Bound by the uneven shares of the tiles (256 workgroups are a multiple of the 128 tiles of 2000 atoms, so each gets the
+// same tile of every second frame, and those of j <= a are empty): CUs busy 38 %, VALU 25 %. 64 frames x 2000 atoms
+// (2.56e8 ordered pairs, 14.7 % within): 0.67 ms; one box of 4000 atoms: 0.041 ms (exact FP64 of every ordered pair, 64
+// absorbers per workgroup: 2.00 ms, 0.377 ms).
 constexpr int PH_WAVES = 16, PH_ROWS = 128, PH_COLS = 256;
 
 template <int KIND>
@@ -282,7 +284,7 @@ __global__ __launch_bounds__(FM_WAVE *PH_WAVES) void k_pair_hist_lds(int natom, 
 // bins (i0, i0 + 1) of potential ipot[j]; its distance moves with pos_j - pos_a. A wavefront takes PG_ROWS atoms a,
 // tests them against 64 atoms j at a time (float coordinates of PG_COLS atoms staged in LDS per workgroup), and
 // evaluates each atom's queue of candidates 64 at a time; the lanes' sums are added in a fixed butterfly: no atomics,
-// the same result on every run. Bound by VALU issue of the float test. 64 frames x 2000 atoms: 0.41 ms; one box of
+// the same result on every run. Bound by VALU issue (82 % busy). 64 frames x 2000 atoms: 0.41 ms; one box of
 // 4000: 0.074 ms (one thread per atom over all j in FP64: 1.15 ms, and 1.32 ms with its 16 workgroups on the chip).
 constexpr int PG_WAVES = 4, PG_ROWS = 4, PG_COLS = 1024;
 
